@@ -504,6 +504,17 @@ int route(tmt_moe* m, hipStream_t s, int T, const uint16_t* X, const uint16_t* W
     return TMT_MOE_OK;
 }
 
+// A combine that finds its slots from the pick table and writes the dispatch
+// tables (the router wrote the picks only).
+void combine_self_dispatch(tmt_moe* m, int T, CombineParams* cp) {
+    cp->self_dispatch = 1;
+    cp->idx = m->idx;
+    DispatchTables& dt = cp->tables;
+    dt.T = T; dt.E = m->desc.experts; dt.K = m->desc.topk; dt.probs = m->probs; dt.lse = m->lse;
+    dt.offsets = m->offsets; dt.counts = m->counts; dt.order = m->order;
+    dt.perm = m->perm; dt.slot_of = m->slot_of; dt.stats = m->stats;
+}
+
 int check_ptrs(const void* const* tab, int n, const char* what, unsigned align = 16) {
     if (!tab) return fail(TMT_MOE_EINVAL, "%s table is NULL", what);
     for (int e = 0; e < n; ++e) {
@@ -606,13 +617,7 @@ int run_forward(tmt_moe* m, hipStream_t s, int T, const uint16_t* X, const uint1
         if (halves) {  // the decode GEMM_DOWN left two fp32 K halves; O is formed here
             cp.part = m->dpart; cp.O_out = m->O; cp.slots = T * K;
         }
-        if (self) {
-            cp.self_dispatch = 1; cp.idx = m->idx;
-            DispatchTables& dt = cp.tables;
-            dt.T = T; dt.E = E; dt.K = K; dt.probs = m->probs; dt.lse = m->lse;
-            dt.offsets = m->offsets; dt.counts = m->counts; dt.order = m->order;
-            dt.perm = m->perm; dt.slot_of = m->slot_of; dt.stats = m->stats;
-        }
+        if (self) combine_self_dispatch(m, T, &cp);
         LAUNCH(TMT_MOE_PH_COMBINE, launch_combine(cp, s));
     }
     m->last_T = T;
@@ -1050,7 +1055,11 @@ int tmt_moe_forward_mxfp4(tmt_moe* m, void* stream, int32_t T, const uint16_t* X
     hipStream_t s = (hipStream_t)stream;
     m->last_T = -1;
     m->last_ln = false;
-    if ((rc = route(m, s, T, X, Wr, logit_bias))) return rc;
+    // Decode-sized batches in the exact format stream the codes with the
+    // skinny kernel; with several tokens the router then writes only the
+    // picks, as in the bf16 decode.
+    const bool self = !is_mx(ds.weight_format) && T <= kSkinnyMaxTokens && E > 1 && T > 1;
+    if ((rc = route(m, s, T, X, Wr, logit_bias, self))) return rc;
     if (T > 0 && is_mx(ds.weight_format)) {
         const int TK = T * K;
         const int64_t srows = (int64_t)ds.max_tokens * K + kMxScalePadRows;
@@ -1102,16 +1111,21 @@ int tmt_moe_forward_mxfp4(tmt_moe* m, void* stream, int32_t T, const uint16_t* X
         up.N = h; up.K = d; up.slots = T * K;
         up.a = X; up.lda = d; up.c = nullptr; up.ldc = h; up.c2 = m->Aact;  // no backward: silu'(U) not kept
         for (int e = 0; e < E; ++e) { up.wq[e] = W_up[e]; up.wsc[e] = W_up_scale[e]; }
-        LAUNCH(TMT_MOE_PH_GEMM_UP, launch_gemm(GEMM_UP_FP4, true, up, s));
+        up.idx = E > 1 ? m->idx : nullptr; up.topk = K; up.self_dispatch = self ? 1 : 0;
+        LAUNCH(TMT_MOE_PH_GEMM_UP, skinny_fp4_fits(up, T) ? launch_skinny_fp4(GEMM_UP_FP4, up, T, s)
+                                                         : launch_gemm(GEMM_UP_FP4, true, up, s));
         GemmParams dn{};
         dn.offsets = m->offsets; dn.order = m->order; dn.perm = m->perm; dn.E = E;
         dn.N = d; dn.K = h; dn.slots = T * K;
         dn.a = m->Aact; dn.lda = h; dn.c = m->O; dn.ldc = d;
         for (int e = 0; e < E; ++e) { dn.wq[e] = W_down[e]; dn.wsc[e] = W_down_scale[e]; }
-        LAUNCH(TMT_MOE_PH_GEMM_DOWN, launch_gemm(GEMM_DOWN_FP4, false, dn, s));
+        dn.idx = up.idx; dn.topk = K; dn.self_dispatch = up.self_dispatch;
+        LAUNCH(TMT_MOE_PH_GEMM_DOWN, skinny_fp4_fits(dn, T) ? launch_skinny_fp4(GEMM_DOWN_FP4, dn, T, s)
+                                                           : launch_gemm(GEMM_DOWN_FP4, false, dn, s));
         CombineParams cp{};
         cp.O = m->O; cp.slot_of = m->slot_of; cp.gate = m->gate;
         cp.Y = Y; cp.beta = beta; cp.T = T; cp.d = d; cp.K = K; cp.silu = 0;
+        if (self) combine_self_dispatch(m, T, &cp);
         LAUNCH(TMT_MOE_PH_COMBINE, launch_combine(cp, s));
     }
     m->last_T = T;

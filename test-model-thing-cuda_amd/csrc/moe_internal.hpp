@@ -177,6 +177,11 @@ constexpr int kSkinnyMaxTokens = 64;
 // p.c, and the combine adds them (CombineParams::part).
 hipError_t launch_skinny_gemm(GemmKind kind, bool dual, const GemmParams& p, int T, hipStream_t s,
                               bool* halves = nullptr);
+// The same for MXFP4 weights (GEMM_UP_FP4 writing SiLU(U) to c2, GEMM_DOWN_FP4):
+// N a multiple of 64, K a multiple of 64. Rows come from offsets / order / perm,
+// or with self_dispatch (T <= kSkinnyMaxTokens) from the pick table in idx.
+bool skinny_fp4_fits(const GemmParams& p, int T);  // whether the forward takes it
+hipError_t launch_skinny_fp4(GemmKind kind, const GemmParams& p, int T, hipStream_t s);
 // One-token decode: GEMM_DOWN of the token's K experts and the combine in
 // one launch. Workgroup b owns output columns 4b .. 4b+3 for all K picks, so
 // the combine needs no other workgroup's results. Needs K <= 8, h % 256 == 0

@@ -28,6 +28,9 @@
 // the [T][K] pick table, from which each wave finds the tokens of its
 // expert's rows itself instead of reading the permutation (a second round
 // trip before the activation loads).
+#include <algorithm>
+#include <cmath>
+
 #include "device_util.hpp"
 #include "dispatch.hpp"
 #include "route_row.hpp"
@@ -631,6 +634,226 @@ size_t stream_lds_rt(bool halves, bool dual, int rb, int nw, int ntile, int spli
     }
 }
 
+// ---------------------------------------------------------- MXFP4 weights --
+// Small batches on MXFP4 experts (GEMM_UP_FP4 / GEMM_DOWN_FP4). The weight
+// stream is a quarter of the bf16 one, so a decode step is bound by the
+// memory round trips of a workgroup (tables, then codes and activations, then
+// the reduction) more than by bytes: every code and scale load of a
+// workgroup's columns is issued at once, and the grid covers the chip in one
+// round. Workgroup: 64 output columns and up to 16 RBP rows of one expert;
+// wave w reduces the 256-element chunks w, w + nw, ... of K (ONE: one chunk
+// per wave). Lane (g, li) holds, per 16-column tile, the codes of
+// k = 256 q + 128 c + 32 g .. + 31 (c = 0, 1) of column li: one 16-byte load
+// and one scale byte each, the four lane groups of a load reading 64
+// contiguous bytes of 16 columns' rows. 64 columns per workgroup make a
+// block's scale bytes one whole 64-byte segment ([K/32][N] layout). The codes
+// are expanded to bf16 in registers (exact, as in gemm.hip) once per chunk
+// for the RBP row blocks that use them.
+// Measured (d = 1024, h = 4096, E = 32, top-4, T = 8; about 92 MB of the
+// picked experts' codes and scales per step), against the 256 x 256 tiles of
+// gemm.hip: UP 62.8 -> 15.6 us, DOWN 102.8 -> 16.7 us, step 169.6 -> 46.1 us.
+constexpr int kFp4Cols = 64;
+constexpr int kFp4Out = 0x7ffffff0;  // buffer offset past every expert (below 2^30 bytes): reads zero
+
+__device__ __forceinline__ uint4 dequant_fp4x8(uint32_t w, float sc) {
+    return make_uint4(__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 0)),
+                      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 1)),
+                      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 2)),
+                      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 3)));
+}
+
+template <int KIND, int NW, int RBP, bool ONE>
+__global__ __launch_bounds__(64 * NW) void skinny_fp4_kernel(GemmParams p, int nrc) {
+    static_assert(KIND == GEMM_UP_FP4 || KIND == GEMM_DOWN_FP4, "MXFP4 forward GEMMs only");
+    constexpr bool kGather = KIND == GEMM_UP_FP4;
+    constexpr int CT = kFp4Cols / 16;
+    __shared__ f32x4 red[CT][NW][64];  // wave partials of one 16-row block
+    __shared__ int s_tok[kGather ? NW : 1][kSkinnyMaxTokens];
+
+    const int nw = (int)blockDim.x >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // Column tiles fastest: workgroup b runs on XCD b % 8, so every expert's
+    // columns spread over the XCDs whatever the routing. In groups of 16
+    // tiles, neighbours share an XCD (their scale bytes share a line).
+    const int ntile = p.N / kFp4Cols;
+    const int j0 = (int)blockIdx.x % ntile, rr = (int)blockIdx.x / ntile;
+    const int tile = ntile % 16 == 0 ? (j0 & ~15) | ((j0 & 7) << 1) | ((j0 >> 3) & 1) : j0;
+    const int n0 = tile * kFp4Cols;
+    // Rows of this workgroup: up to RB rows of one expert, from slot row0 on
+    // (the expert's rows base .. base + rows - 1).
+    constexpr int RB = 16 * RBP;
+    const bool self = p.self_dispatch != 0;
+    int e, row0, rows, base = 0;
+    int ent[kPickGroups];
+    if (self) {
+        load_picks(p, lane, ent);
+        e = rr / nrc;
+        base = (rr % nrc) * RB;
+        expert_span(ent, p.slots, e, row0, rows);
+        // an expert without rows here is left before its codes are requested
+        // (at T = 8 a third of 32 experts are empty)
+        if (rows <= base) return;
+        row0 += base;
+        rows = min(rows - base, RB);
+    } else {
+        const ExpertTiles et = expert_tiles<RB>(p.offsets, p.E, lane);
+        if (!expert_tile<RB>(et, rr, e, row0, rows)) return;
+    }
+    const int nrb = (rows + 15) >> 4;
+    const int g = lane >> 4, li = lane & 15;
+    const int K = p.K, N = p.N, nchunk = (K + 255) >> 8;
+    const __amdgpu_buffer_rsrc_t cr = weight_rsrc(reinterpret_cast<const uint16_t*>(p.wq[e]), N * (K / 2));
+    const __amdgpu_buffer_rsrc_t sr = weight_rsrc(reinterpret_cast<const uint16_t*>(p.wsc[e]), (K / 32) * N);
+    struct Chunk {
+        uint4 code[CT][2];
+        uint32_t scale[CT][2];
+    };
+    auto load_chunk = [&](int q, Chunk& w) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int k0 = 256 * q + 128 * c + 32 * g;
+            const bool in = k0 < K;  // K is a multiple of 64: a 32-element block is inside or outside as a whole
+#pragma unroll
+            for (int t = 0; t < CT; ++t) {
+                const int n = n0 + 16 * t + li;
+                w.code[t][c] = ld16_buf(cr, in ? n * (K / 2) + k0 / 2 : kFp4Out);
+                w.scale[t][c] = __builtin_amdgcn_raw_buffer_load_b8(sr, in ? (k0 / 32) * N + n : kFp4Out, 0, 0);
+            }
+        }
+    };
+    Chunk cur;
+    load_chunk(wave, cur);
+    if constexpr (kGather) {
+        if (self) expert_tokens(ent, p.slots, p.topk, e, lane, kSkinnyMaxTokens, s_tok[wave]);
+    }
+    // this lane's activation row in each row block (rows past the expert's
+    // count read its first row and enter as zeros)
+    const uint16_t* ar[RBP];
+    bool ok[RBP];
+#pragma unroll
+    for (int i = 0; i < RBP; ++i) {
+        const int m = 16 * i + li;
+        ok[i] = m < rows;
+        const int mm = ok[i] ? m : 0;
+        const int srow = !kGather ? row0 + mm : (self ? s_tok[wave][base + mm] : p.perm[row0 + mm]);
+        ar[i] = p.a + (int64_t)srow * p.lda;
+    }
+    f32x4 acc[RBP][CT];
+#pragma unroll
+    for (int i = 0; i < RBP; ++i)
+#pragma unroll
+        for (int t = 0; t < CT; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto mul_chunk = [&](int q, const Chunk& w) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int k0 = 256 * q + 128 * c + 32 * g;
+            const int kk = k0 < K ? k0 : 0;
+            uint4 av[RBP][4];
+#pragma unroll
+            for (int i = 0; i < RBP; ++i) {
+                if (i >= nrb) break;  // uniform
+#pragma unroll
+                for (int j = 0; j < 4; ++j) av[i][j] = ld16(ar[i] + kk + 8 * j);
+                if (!ok[i] || k0 >= K) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) av[i][j] = make_uint4(0, 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < CT; ++t) {
+                // e8m0: 2^(s - 127); s = 0 is the subnormal 2^-127
+                const uint32_t s8 = w.scale[t][c];
+                const float sc = __uint_as_float(s8 == 0 ? 0x00400000u : (s8 << 23));
+                const uint32_t cw[4] = {w.code[t][c].x, w.code[t][c].y, w.code[t][c].z, w.code[t][c].w};
+                uint4 wb[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) wb[j] = dequant_fp4x8(cw[j], sc);
+#pragma unroll
+                for (int i = 0; i < RBP; ++i) {
+                    if (i >= nrb) break;  // uniform
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[i][t] = mfma16(wb[j], av[i][j], acc[i][t]);
+                }
+            }
+        }
+    };
+    if constexpr (ONE) {
+        mul_chunk(wave, cur);
+    } else {
+        // the next chunk's codes are requested before this one is multiplied
+        for (int q = wave; q < nchunk; q += nw) {
+            Chunk nxt;
+            load_chunk(min(q + nw, nchunk), nxt);  // chunk nchunk: past K, zeros
+            __builtin_amdgcn_sched_barrier(0);
+            mul_chunk(q, cur);
+            cur = nxt;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < RBP; ++i) {
+        if (i >= nrb) break;  // uniform
+        if (i > 0) __syncthreads();
+        // acc[i][t][r] = C[row 16 i + li][column n0 + 16 t + 4 g + r]
+#pragma unroll
+        for (int t = 0; t < CT; ++t) red[t][wave][lane] = acc[i][t];
+        __syncthreads();
+        // unit o: column tile o / 64, lane o % 64 of the MFMA layout (one row,
+        // four columns); the wave partials are added in wave order
+        for (int o = tid; o < CT * 64; o += (int)blockDim.x) {
+            const int t = o >> 6, sl = o & 63;
+            const int row = 16 * i + (sl & 15);
+            if (row >= rows) continue;
+            f32x4 v = red[t][0][sl];
+            for (int w2 = 1; w2 < nw; ++w2) v += red[t][w2][sl];
+            if constexpr (kGather) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = silu_fast(v[r]);
+            }
+            uint16_t* C = kGather ? p.c2 : reinterpret_cast<uint16_t*>(p.c);
+            *reinterpret_cast<uint2*>(C + (int64_t)(row0 + row) * p.ldc + n0 + 16 * t + 4 * (sl >> 4)) =
+                make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+        }
+    }
+}
+
+template <int KIND, int RBP>
+hipError_t launch_fp4_rows(const GemmParams& p, int T, hipStream_t s) {
+    constexpr int RB = 16 * RBP;
+    const int nchunk = (p.K + 255) / 256;
+    const int most = RBP == 1 && nchunk <= 16 ? 16 : 8;  // waves (16 only with one chunk each: 128 VGPRs)
+    const int nw = std::min(nchunk, most);
+    // self_dispatch: the expert's row blocks by index; otherwise the list of
+    // (expert, row block) from the offsets, at most slots / RB + E entries
+    const int nrc = (std::min(T, p.slots) + RB - 1) / RB;
+    const int64_t blocks = p.self_dispatch ? (int64_t)p.E * nrc
+                                           : std::min<int64_t>((int64_t)p.slots / RB + p.E, p.slots);
+    const int64_t grid = (int64_t)(p.N / kFp4Cols) * blocks;
+    if (grid > 0x7fffffff) return hipErrorInvalidValue;
+    const unsigned gr = (unsigned)grid;
+    const dim3 block(64 * nw);
+    if (nchunk > most) skinny_fp4_kernel<KIND, 8, RBP, false><<<gr, block, 0, s>>>(p, nrc);
+    else if (nw > 8) {
+        if constexpr (RBP == 1) skinny_fp4_kernel<KIND, 16, 1, true><<<gr, block, 0, s>>>(p, nrc);
+    } else if (nw > 4) skinny_fp4_kernel<KIND, 8, RBP, true><<<gr, block, 0, s>>>(p, nrc);
+    else skinny_fp4_kernel<KIND, 4, RBP, true><<<gr, block, 0, s>>>(p, nrc);
+    return hipGetLastError();
+}
+template <int KIND>
+hipError_t launch_fp4_kind(const GemmParams& p, int T, hipStream_t s) {
+    // Rows per workgroup. self_dispatch has a workgroup for every row block
+    // an expert could have, so one block takes all T <= 64 rows (T = 64, 32
+    // experts, top-4: 69 us a step with 64 rows, 85 with 16 and four times the
+    // workgroups, most of them empty). From the offsets only real blocks are
+    // launched: 16 rows where experts have about that many (T = 65: 70 us,
+    // 74 with 32 rows), else 32, which expand each code once for two blocks
+    // (T = 512: 164 us, 185 with 16 and 173 with 64 rows).
+    if (p.self_dispatch) {
+        if (T <= 16) return launch_fp4_rows<KIND, 1>(p, T, s);
+        return T <= 32 ? launch_fp4_rows<KIND, 2>(p, T, s) : launch_fp4_rows<KIND, 4>(p, T, s);
+    }
+    return p.slots <= 16 * p.E ? launch_fp4_rows<KIND, 1>(p, T, s) : launch_fp4_rows<KIND, 2>(p, T, s);
+}
 
 }  // namespace
 
@@ -780,6 +1003,32 @@ hipError_t launch_skinny_gemm(GemmKind kind, bool dual, const GemmParams& p, int
         return dual ? launch_rb<GEMM_UP, true>(rb, p, nexp, grid, s)
                     : launch_rb<GEMM_UP, false>(rb, p, nexp, grid, s);
     return launch_rb<GEMM_DOWN, false>(rb, p, nexp, grid, s);
+}
+
+// Whether a forward GEMM over MXFP4 weights streams its codes (skinny) rather
+// than running 256 x 256 tiles. Decode batches always do; above them the two
+// times are estimated from what they measured on one MI355X (us): a round of
+// tiles costs 12 + 1.6 per 64 of K whatever its rows hold, the stream 2 N K
+// operations per routed row at 0.28 PFLOP/s. Row tiles: one per expert up to
+// a mean of 128 rows, then half of the last one is empty on average. E.g.
+// (us a step, tiles / stream) d = 1024, h = 4096, E = 32, top-4: T = 256
+// 210 / 112, T = 1024 226 / 268; d = 512, h = 2048, E = 8, top-2: T = 512
+// 91 / 43, T = 4096 127 / 130; the two GEMMs of a step decide on their own.
+bool skinny_fp4_fits(const GemmParams& p, int T) {
+    if (T <= kSkinnyMaxTokens) return true;
+    const double mtiles = std::max<double>(std::min(p.E, p.slots), p.slots / 256.0 + 0.5 * p.E);
+    const double rounds = std::ceil(mtiles * ((p.N + 255) / 256) / cu_count());
+    return 2.0 * p.slots * p.N * p.K / 0.28e9 < rounds * (12.0 + 1.6 * p.K / 64);
+}
+
+hipError_t launch_skinny_fp4(GemmKind kind, const GemmParams& p, int T, hipStream_t s) {
+    if (p.slots <= 0 || T <= 0) return hipSuccess;
+    if (p.N % kFp4Cols != 0 || p.N <= 0 || p.K % 64 != 0 || p.K <= 0 || (int64_t)p.N * p.K / 2 >= kFp4Out)
+        return hipErrorInvalidValue;
+    if (p.self_dispatch && (p.idx == nullptr || T > kSkinnyMaxTokens)) return hipErrorInvalidValue;
+    if (kind == GEMM_UP_FP4) return launch_fp4_kind<GEMM_UP_FP4>(p, T, s);
+    if (kind == GEMM_DOWN_FP4) return launch_fp4_kind<GEMM_DOWN_FP4>(p, T, s);
+    return hipErrorInvalidValue;
 }
 
 }  // namespace tmt

@@ -92,6 +92,32 @@ def test_mxfp4_against_oracle(orc, fmt, T, d, E, K, h):
     assert err <= TOL
 
 
+@pytest.mark.parametrize("T,d,E,K,h", [
+    (1, 1024, 32, 4, 4096),    # one token: tables from the router, one row per expert, 16 waves in DOWN
+    (64, 1024, 32, 4, 256),    # the largest decode batch
+    (8, 320, 64, 8, 64),       # 64 experts; K = 320 (a partial chunk) and K = 64 (a quarter of one)
+    (33, 256, 2, 2, 4352),     # 33 rows per expert (three row blocks); DOWN over 17 chunks on 16 waves
+    (40, 192, 1, 1, 1088),     # one expert: slot = token, five waves in DOWN
+    (2, 2048, 4, 1, 2304),     # 8 waves in UP, 9 in DOWN
+])
+def test_mxfp4_decode_against_oracle(orc, T, d, E, K, h):
+    """Decode batches of the exact format: the weight-streaming kernel's
+    tables, statistics and output. The weights expand exactly to bf16, so Y
+    differs from the oracle's only by the bf16 rounding of the hidden
+    activations, expert outputs and Y (2^-9 relative each, three of them:
+    under 6e-3 relative L2)."""
+    say(f"mxfp4 decode T={T} d={d} E={E} K={K} h={h}")
+    case = make_case(T, d, E, K, h, seed=31 + T)
+    Y0 = bf16_bits(np.random.default_rng(T).standard_normal((T, d)).astype(np.float32))
+    g, wu, wd = run_fp4(case, K, h, beta=1.0, Y0=Y0)
+    r = orc.forward(case["X"], case["Wr"], wu, wd, K, h, Y_in=Y0, beta=1.0)
+    assert np.array_equal(g["idx"], r["idx"]) and np.array_equal(g["perm"], r["perm"])
+    assert np.array_equal(g["offsets"], r["offsets"]) and np.array_equal(g["slot_of"], r["slot_of"])
+    err = rel_l2(g["Y"], r["Y"])
+    say(f"  Y rel-L2 {err:.2e}")
+    assert err <= 6e-3
+
+
 def test_mxfp4_mx_tracks_exact_format(orc):
     """The MX format differs from the exact-product format only by the
     activations' two-term MXFP6 rounding: well under the c5 tolerance."""
