@@ -148,16 +148,9 @@ __device__ __forceinline__ uint4 dequant8(uint32_t w, uint32_t scale) {
                       __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, sc, 3)));
 }
 
-// Streaming (non-temporal) 16-byte accesses for the epilogue: outputs are
-// written once and read by a later kernel, so they should not displace the
+// Streaming 16-byte accesses for the epilogue: outputs are written once
+// (st16_nt) and read by a later kernel, so they should not displace the
 // operand tiles the other workgroups are reusing from L2.
-typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void st16_nt(void* p, uint4 v) {
-    __builtin_nontemporal_store(u32x4_t{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4_t*>(p));
-}
-__device__ __forceinline__ void st16_nt(void* p, f32x4 v) {
-    __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(p));
-}
 __device__ __forceinline__ uint4 ld16_nt(const uint16_t* p) {
     const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
     return make_uint4(v[0], v[1], v[2], v[3]);

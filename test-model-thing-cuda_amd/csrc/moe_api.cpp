@@ -132,7 +132,7 @@ struct tmt_moe {
     float *dlogits, *dwr_partial;
     // LayerNorm in front of the block (tmt_moe_forward_ln / tmt_moe_backward_ln)
     uint16_t *H, *dH;
-    float *ln_mean, *ln_rstd, *ln_partial, *ln_partial2;
+    float *ln_mean, *ln_rstd, *ln_partial;
     int last_T = -1;
     bool last_ln = false;  // the last forward was tmt_moe_forward_ln
     // per-kernel event timing (tmt_moe_set_profiling)
@@ -281,9 +281,8 @@ Sizes plan(const tmt_moe_desc* user, tmt_moe* m) {
     size_t o_xq = mx ? W.add(mx_codes_bytes(TK, D)) : 0, o_xqs = mx ? W.add(mx_scales_bytes(TK, D)) : 0;
     size_t o_aq = mx ? W.add(mx_codes_bytes(TK, h)) : 0, o_aqs = mx ? W.add(mx_scales_bytes(TK, h)) : 0;
     size_t o_wpl = d->weight_format == TMT_MOE_WEIGHTS_MXFP4_MX ? W.add((size_t)E * h * D) : 0;
-    const int64_t ln_rows = std::max(scatter_blocks((int)T), ln_chunks((int)T));
+    const int64_t ln_rows = std::max(scatter_blocks_max((int)T), ln_chunks((int)T));
     size_t o_lnp = bwd ? W.add((size_t)ln_rows * 2 * D * 4) : 0;
-    size_t o_lnp2 = bwd ? W.add((size_t)colsum_groups((int)ln_rows) * 2 * D * 4) : 0;
     // zero-padded operand copies of a handle whose widths are not multiples
     // of 64 (transient: every call fills the ones it reads)
     const bool pad = is_padded(*user);
@@ -346,7 +345,6 @@ Sizes plan(const tmt_moe_desc* user, tmt_moe* m) {
         m->ln_rstd = (float*)(a + o_rstd);
         m->dH = bwd ? (uint16_t*)(w + o_dH) : nullptr;
         m->ln_partial = bwd ? (float*)(w + o_lnp) : nullptr;
-        m->ln_partial2 = bwd ? (float*)(w + o_lnp2) : nullptr;
         m->nblk_max = (int)nblk;
         m->padded = pad;
         if (pad) {
@@ -734,10 +732,10 @@ int run_backward(tmt_moe* m, hipStream_t s, const uint16_t* dY, const uint16_t* 
         // reference's (moe.cu:486-487).
         LAUNCH(TMT_MOE_PH_ROUTER_DW, launch_zero_f32(dWr, d, s));
     }
-    // Without the LayerNorm the scatter's launch also runs the router weight
-    // gradient's second pass (one launch fewer).
+    // The scatter's launch also runs the router weight gradient's second pass
+    // (one launch fewer).
     RouterDwParams rw{};
-    const bool dw_in_scatter = E > 1 && T > 0 && ln == nullptr;
+    const bool dw_in_scatter = E > 1 && T > 0;
     if (E > 1) {
         // With T == 0 the partial pass sums no rows and writes zeros.
         rw.dlogits = m->dlogits; rw.X = X; rw.T = T; rw.d = d; rw.E = E;
@@ -759,8 +757,8 @@ int run_backward(tmt_moe* m, hipStream_t s, const uint16_t* dY, const uint16_t* 
         LAUNCH(TMT_MOE_PH_SCATTER, launch_scatter(sc, s));
     }
     if (ln_fused) {
-        LAUNCH(TMT_MOE_PH_NORM_BWD, launch_colsum(m->ln_partial, T > 0 ? scatter_blocks(T) : 0, 2 * d,
-                                                  m->ln_partial2, d, d, ln->dGamma, ln->dBeta, s));
+        LAUNCH(TMT_MOE_PH_NORM_BWD, launch_colsum(m->ln_partial, T > 0 ? scatter_blocks(T) : 0, 2 * d, d, d,
+                                                  ln->dGamma, ln->dBeta, s));
     } else if (ln) {
         // the caller's S / dS rows have the caller's width; dX (the gradient
         // at H) has the internal one
@@ -768,7 +766,7 @@ int run_backward(tmt_moe* m, hipStream_t s, const uint16_t* dY, const uint16_t* 
         lp.S = ln->S; lp.gamma = ln->gamma; lp.T = T; lp.d = m->user.d;
         lp.lds = m->user.d; lp.ldh = d;
         lp.mean = m->ln_mean; lp.rstd = m->ln_rstd; lp.dH = dX; lp.dS = ln->dS;
-        lp.partial = m->ln_partial; lp.partial2 = m->ln_partial2; lp.dgamma = ln->dGamma; lp.dbeta = ln->dBeta;
+        lp.partial = m->ln_partial; lp.dgamma = ln->dGamma; lp.dbeta = ln->dBeta;
         LAUNCH(TMT_MOE_PH_NORM_BWD, launch_ln_bwd(lp, s));
     }
     return TMT_MOE_OK;
@@ -780,13 +778,14 @@ int check_ln_shape(int32_t T, int32_t d) {
     return TMT_MOE_OK;
 }
 
-// Workspace of the standalone LayerNorm backward, in floats: chunk partials,
-// then (from *level1_off, 256-byte aligned) the level-1 column sums.
-size_t ln_workspace_floats(int32_t T, int32_t d, size_t* level1_off) {
+// Workspace of the standalone LayerNorm backward, in floats: the chunk
+// partials, and a row pair per 64 chunks that callers' buffers have always
+// held (the size, and with it the shapes the no-allocation entry point
+// takes, is part of the interface).
+size_t ln_workspace_floats(int32_t T, int32_t d) {
     const size_t nch = (size_t)ln_chunks(T), pw = (size_t)ln_width4(d);
     const size_t off = (nch * 2 * pw + 63) & ~size_t(63);
-    *level1_off = off;
-    return off + (size_t)colsum_groups((int)nch) * 2 * pw;
+    return off + (nch + 63) / 64 * 2 * pw;
 }
 
 int check_ln_backward_args(int32_t T, int32_t d, const uint16_t* S, const uint16_t* dH, const float* gamma,
@@ -803,17 +802,15 @@ int check_ln_backward_args(int32_t T, int32_t d, const uint16_t* S, const uint16
     return TMT_MOE_OK;
 }
 
-// The LayerNorm backward's launches over a workspace at `ws` (chunk
-// partials, then the level-1 column sums from float offset `level1_off`).
-// Every workspace element the kernels read is written by them first.
+// The LayerNorm backward's launches over a workspace at `ws` (the chunk
+// partials). Every workspace element the kernels read is written by them first.
 int run_ln_backward(hipStream_t s, int32_t T, int32_t d, const uint16_t* S, const uint16_t* dH,
                     const float* gamma, const float* mean, const float* rstd, uint16_t* dS, float* dGamma,
-                    float* dBeta, float* ws, size_t level1_off) {
+                    float* dBeta, float* ws) {
     LayerNormParams p{};
     p.S = S; p.gamma = gamma; p.T = T; p.d = d; p.lds = d; p.ldh = d; p.mean = const_cast<float*>(mean);
     p.rstd = const_cast<float*>(rstd); p.dH = dH; p.dS = dS;
     p.partial = ws;
-    p.partial2 = ws + level1_off;
     p.dgamma = dGamma; p.dbeta = dBeta;
     HIP_TRY(launch_ln_bwd(p, s));
     return TMT_MOE_OK;
@@ -1271,8 +1268,7 @@ int tmt_moe_layernorm_workspace_size(int32_t T, int32_t d, size_t* bytes) {
     int rc = check_ln_shape(T, d);
     if (rc) return rc;
     if (!bytes) return fail(TMT_MOE_EINVAL, "bytes is NULL");
-    size_t off;
-    *bytes = ln_workspace_floats(T, d, &off) * 4;
+    *bytes = ln_workspace_floats(T, d) * 4;
     return TMT_MOE_OK;
 }
 
@@ -1296,14 +1292,13 @@ int tmt_moe_layernorm_backward(void* stream, int32_t T, int32_t d, const uint16_
                                float* dGamma, float* dBeta, void* workspace, size_t workspace_bytes) {
     int rc = check_ln_backward_args(T, d, S, dH, gamma, mean, rstd, dS, dGamma, dBeta);
     if (rc) return rc;
-    size_t off;
-    const size_t need = ln_workspace_floats(T, d, &off) * 4;
+    const size_t need = ln_workspace_floats(T, d) * 4;
     if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
         return fail(TMT_MOE_EINVAL, "workspace must be a 256-byte aligned device pointer");
     if (workspace_bytes < need)
         return fail(TMT_MOE_EINVAL, "workspace of %zu bytes is smaller than the %zu bytes needed", workspace_bytes, need);
     return run_ln_backward((hipStream_t)stream, T, d, S, dH, gamma, mean, rstd, dS, dGamma, dBeta,
-                           static_cast<float*>(workspace), off);
+                           static_cast<float*>(workspace));
 }
 
 int tmt_moe_layernorm_backward_noalloc(void* stream, int32_t T, int32_t d, const uint16_t* S,
@@ -1311,15 +1306,14 @@ int tmt_moe_layernorm_backward_noalloc(void* stream, int32_t T, int32_t d, const
                                        const float* rstd, uint16_t* dS, float* dGamma, float* dBeta) {
     int rc = check_ln_backward_args(T, d, S, dH, gamma, mean, rstd, dS, dGamma, dBeta);
     if (rc) return rc;
-    size_t off;
-    const size_t need = ln_workspace_floats(T, d, &off) * 4;
+    const size_t need = ln_workspace_floats(T, d) * 4;
     if (need > kNoAllocScratchBytes)
         return fail(TMT_MOE_EINVAL,
                     "T=%d, d=%d needs %zu bytes of scratch, more than the %zu bytes this entry point holds",
                     T, d, need, kNoAllocScratchBytes);
     float* ws = nullptr;
     if ((rc = scratch_on_current_device(&ws))) return rc;
-    return run_ln_backward((hipStream_t)stream, T, d, S, dH, gamma, mean, rstd, dS, dGamma, dBeta, ws, off);
+    return run_ln_backward((hipStream_t)stream, T, d, S, dH, gamma, mean, rstd, dS, dGamma, dBeta, ws);
 }
 
 int tmt_moe_f32_to_bf16(void* stream, const float* in, uint16_t* out, int64_t n) {

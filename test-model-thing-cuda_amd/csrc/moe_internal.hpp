@@ -356,13 +356,15 @@ struct ScatterParams {
     float* ln_partial;       // [scatter_blocks(T)][2][d] per-block dgamma / dbeta sums
     // Pass 2 of the router weight gradient (the per-output sum over pass 1's
     // chunks) run by extra workgroups of the same launch (dw.partial !=
-    // nullptr; only without the LayerNorm): the two are independent, and
-    // one launch fewer shortens a small backward.
+    // nullptr): the two are independent, and one launch fewer shortens a
+    // small backward.
     RouterDwParams dw;
 };
 constexpr int kLnFusedMaxD = 2048;
-constexpr int kScatterRows = 64;  // rows per scatter workgroup (router or LayerNorm variants)
+// Workgroups (and ln_partial rows) of the scatter with the LayerNorm backward
+// fused, and the most of any T <= max_tokens.
 int scatter_blocks(int T);
+int scatter_blocks_max(int max_tokens);
 hipError_t launch_scatter(const ScatterParams& p, hipStream_t s);
 
 // p[0, n) = 0 with a kernel (no memset node, so the call can be captured).
@@ -393,7 +395,6 @@ struct LayerNormParams {
     const uint16_t* dH;      // [T][ldh] bf16 gradient at H (backward)
     uint16_t* dS;            // [T][lds] bf16 (backward)
     float* partial;          // [ln_chunks(T)][2][ln_width4(d)] dgamma / dbeta chunk sums
-    float* partial2;         // [colsum_groups(ln_chunks(T))][2][ln_width4(d)] (level-1 sums)
     float* dgamma;           // [d]
     float* dbeta;            // [d]
 };
@@ -404,11 +405,9 @@ hipError_t launch_ln_fwd(const LayerNormParams& p, hipStream_t s);
 hipError_t launch_ln_bwd(const LayerNormParams& p, hipStream_t s);
 // Fixed-order column sums of in [nrows][ncols] (ncols % 4 == 0): columns
 // [0, split) to out_lo, [split, ncols) to out_hi, each of which receives its
-// first `width` columns (width <= split, ncols - split); scratch holds
-// [colsum_groups(nrows)][ncols] level-1 sums.
-int colsum_groups(int nrows);
-hipError_t launch_colsum(const float* in, int nrows, int ncols, float* scratch, int split, int width,
-                         float* out_lo, float* out_hi, hipStream_t s);
+// first `width` columns (width <= split, ncols - split).
+hipError_t launch_colsum(const float* in, int nrows, int ncols, int split, int width, float* out_lo,
+                         float* out_hi, hipStream_t s);
 
 // Zero-padded copies between a caller's matrices and the internal ones of a
 // handle whose width is not a multiple of 64: dst[r][c] = src[r][c] for

@@ -540,6 +540,11 @@ constexpr int kRedOnWrExperts = 12;  // E*d*2 bytes of Wr hold the 3*2*d floats
 template <bool ROUTER, int NI, bool WLDS>
 __global__ __launch_bounds__(kThreads) void scatter_kernel(ScatterParams p, int rows_per_block) {
     extern __shared__ uint4 smem_w[];
+    const int nrow_blocks = (p.T + rows_per_block - 1) / rows_per_block;
+    if ((int)blockIdx.x >= nrow_blocks) {  // the router weight gradient's pass 2
+        router_dw_reduce_block(p.dw, blockIdx.x - nrow_blocks);
+        return;
+    }
     constexpr int NR = NI > 0 ? NI : 1;
     constexpr bool STAGE = ROUTER && WLDS;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -887,6 +892,11 @@ __global__ __launch_bounds__(kThreads) void scatter_rows_kernel(ScatterParams p,
 template <int K, int NI, bool WLDS>
 __global__ __launch_bounds__(kThreads) void scatter_ln2_kernel(ScatterParams p, int rows_per_block) {
     extern __shared__ uint4 smem_w[];
+    const int nrow_blocks = (p.T + rows_per_block - 1) / rows_per_block;
+    if ((int)blockIdx.x >= nrow_blocks) {  // the router weight gradient's pass 2
+        router_dw_reduce_block(p.dw, blockIdx.x - nrow_blocks);
+        return;
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int d = p.d, E = p.E;
     const int rbeg = blockIdx.x * rows_per_block;
@@ -1064,16 +1074,34 @@ __global__ __launch_bounds__(kThreads) void scatter_ln2_kernel(ScatterParams p, 
 
 }  // namespace
 
+// Rows per workgroup of the LayerNorm variants: 64, fewer while that keeps
+// the grid under kScatterLnBlocks workgroups. A workgroup's waves walk their rows in
+// a chain of load round trips, so a small batch finishes sooner on many short
+// workgroups: T = 1024, d = 256 took 19.9 us on 16 workgroups of 64 rows, 6.0
+// on 128 of 8 with the router gradient's second pass (3 us) riding along. The
+// block's step at T = 4096, d = 1024, E = 16: 239 us below 128 workgroups,
+// 230 below 256, 226.5 below 512 and below 1024.
+constexpr int kScatterLnRows = 64, kScatterLnRowsMin = 8, kScatterLnBlocks = 512;
+static int scatter_ln_rows(int T) {
+    int rows = kScatterLnRows;
+    while (rows > kScatterLnRowsMin && (T + rows - 1) / rows < kScatterLnBlocks) rows /= 2;
+    return rows;
+}
 int scatter_blocks(int T) {
-    const int b = (T + kScatterRows - 1) / kScatterRows;
+    const int rows = scatter_ln_rows(T), b = (T + rows - 1) / rows;
     return b < 1 ? 1 : b;
+}
+// Below 64 rows per workgroup the grid stays under 2 * kScatterLnBlocks.
+int scatter_blocks_max(int max_tokens) {
+    const int full = (max_tokens + kScatterLnRows - 1) / kScatterLnRows;
+    const int few = std::min((max_tokens + kScatterLnRowsMin - 1) / kScatterLnRowsMin, 2 * kScatterLnBlocks);
+    return std::max(1, std::max(full, few));
 }
 
 template <bool ROUTER, bool WLDS>
 hipError_t launch_scatter_ni(const ScatterParams& p, int ni, int rows, size_t lds, hipStream_t s) {
-    const int grid = (p.T + rows - 1) / rows;
+    const int grid = (p.T + rows - 1) / rows + (p.dw.partial != nullptr ? router_dw_reduce_blocks(p.dw) : 0);
     switch (ni) {
-        case 0: scatter_kernel<ROUTER, 0, WLDS><<<grid, kThreads, lds, s>>>(p, rows); break;
         case 1: scatter_kernel<ROUTER, 1, WLDS><<<grid, kThreads, lds, s>>>(p, rows); break;
         case 2: scatter_kernel<ROUTER, 2, WLDS><<<grid, kThreads, lds, s>>>(p, rows); break;
         case 3: scatter_kernel<ROUTER, 3, WLDS><<<grid, kThreads, lds, s>>>(p, rows); break;
@@ -1190,11 +1218,11 @@ hipError_t launch_zero_f32(float* p, int64_t n, hipStream_t s) {
 
 hipError_t launch_scatter(const ScatterParams& p, hipStream_t s) {
     if (p.T <= 0) return hipSuccess;
-    if (p.dw.partial != nullptr && (p.ln_S != nullptr || p.dw.nchunks < 1)) return hipErrorInvalidValue;
+    if (p.dw.partial != nullptr && p.dw.nchunks < 1) return hipErrorInvalidValue;
     const bool router = p.dlogits != nullptr && p.E > 1;
     const bool ln = p.ln_S != nullptr;
     if (ln && p.d > kLnFusedMaxD) return hipErrorInvalidValue;
-    const int rows = (router || ln) ? kScatterRows : 4;
+    const int rows = scatter_ln_rows(p.T);  // LayerNorm variants
     const bool wlds = router && router_wr_in_lds(p.E, p.d);  // Wr staged in LDS
     const size_t wr_lds = wlds ? (size_t)p.E * p.d * 2 : 0;
     size_t lds = router ? wr_lds + (size_t)rows * p.E * 4 : 0;
@@ -1232,7 +1260,7 @@ hipError_t launch_scatter(const ScatterParams& p, hipStream_t s) {
     if (!router) return launch_scatter_ni<false, false>(p, ni, rows, lds, s);
     if (p.K <= 4 && ni <= 2) {
         // two rows per wave in flight (scatter_ln2_kernel)
-        const int grid = (p.T + rows - 1) / rows;
+        const int grid = (p.T + rows - 1) / rows + (p.dw.partial != nullptr ? router_dw_reduce_blocks(p.dw) : 0);
 #define TMT_LN2(KK, NN)                                                                                    \
     if (p.K == KK && ni == NN) {                                                                          \
         if (wlds) scatter_ln2_kernel<KK, NN, true><<<grid, kThreads, lds, s>>>(p, rows);                   \

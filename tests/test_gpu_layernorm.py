@@ -347,6 +347,21 @@ def test_c3_full_size_layernorm_block(orc):
         assert err <= REL_L2, f"{n} rel-L2 {err:.3e}"
 
 
+@pytest.mark.parametrize("T,d", [
+    (9000, 1024),  # output beyond the L2s: non-temporal row stores; the last chunk of 512 rows partial
+    (4100, 2304),  # the same with rows read twice (more than 2048 columns)
+    (1100, 1250),  # unaligned rows of three register pieces, three chunks
+    (513, 2050),   # unaligned rows read twice; a chunk of one row
+    (600, 5),      # rows shorter than one 8-element piece
+    (70, 9),       # one full piece and a tail of one element
+])
+def test_standalone_layernorm_row_forms(orc, T, d):
+    """The row forms of the forward and of the one-launch backward (register
+    pieces or read twice, aligned or not, streamed out or not), held to the
+    bounds of the test above."""
+    test_standalone_layernorm_against_oracle(orc, T, d)
+
+
 @pytest.mark.parametrize("T,d,E,norm_launches", [
     (300, 256, 4, 0),     # routed batch: the router normalises its rows itself
     (2100, 2048, 12, 0),  # the widest fused row (4 chunks of 512 per lane)
