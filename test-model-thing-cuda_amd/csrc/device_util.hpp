@@ -109,9 +109,6 @@ typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void st16_nt(void* p, uint4 v) {
     __builtin_nontemporal_store(u32x4_t{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4_t*>(p));
 }
-__device__ __forceinline__ void st16_nt(void* p, f32x4 v) {
-    __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(p));
-}
 
 // SiLU and its derivative (reference tmt-cuda/src/common.h:15-24) with the
 // hardware exp2 / reciprocal: x * sigmoid(x), g*s*(1 + x(1 - s)).

@@ -151,6 +151,7 @@ __device__ __forceinline__ uint4 dequant8(uint32_t w, uint32_t scale) {
 // Streaming 16-byte accesses for the epilogue: outputs are written once
 // (st16_nt) and read by a later kernel, so they should not displace the
 // operand tiles the other workgroups are reusing from L2.
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ uint4 ld16_nt(const uint16_t* p) {
     const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
     return make_uint4(v[0], v[1], v[2], v[3]);
@@ -387,10 +388,12 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
         e = p.order[ei];
         kbeg = p.offsets[e];
         kend = p.offsets[e + 1];
-        mlim = min(BM, p.M - mt * BM);
+        // the outputs may be narrower than the operands' padded widths (by
+        // less than 64, so every tile keeps a row and a column)
+        mlim = min(BM, p.m_out - mt * BM);
     }
     const int col0 = nt * BN;                // the tile's first output column
-    const int nlim = min(BN, p.N - col0);  // valid output columns in this tile
+    const int nlim = min(BN, (Tr::group_k ? p.n_out : p.N) - col0);  // valid output columns in this tile
     const int nk = (kend - kbeg + BK - 1) / BK;
 
     // ---- DMA addressing -----------------------------------------------------
@@ -887,7 +890,11 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
                 const int n = nbase + cl * 4;
                 if (m >= mlim || n >= nlim) continue;
                 const f32x4 v = *reinterpret_cast<const f32x4*>(stage_f + rr * WTN + ((cl ^ (rr & (CH - 1))) * 4));
-                st16_nt(C + (int64_t)(mt * BM + m) * p.ldc + col0 + n, v);
+                float* o = C + (int64_t)(mt * BM + m) * p.ldc + col0 + n;
+                // rows of any width: 16-byte stores at any float's address
+                if (n + 4 <= nlim) __builtin_nontemporal_store(v, reinterpret_cast<f32x4_any*>(o));
+                else
+                    for (int t = 0; t < nlim - n; ++t) o[t] = v[t];
             }
         }
         __syncthreads();
@@ -1032,6 +1039,8 @@ hipError_t launch_gemm_tile(GemmKind kind, bool dual, const GemmParams& p, GemmT
     int64_t gsz = 32;  // tiles per group (weight-gradient GEMMs on 256 columns: 16)
     if (group_k) {
         if (p.M % 8 != 0 || p.M <= 0) return hipErrorInvalidValue;
+        if (p.m_out > p.M || p.n_out > p.N || p.M - p.m_out >= 64 || p.N - p.n_out >= 64 || p.ldc < p.n_out)
+            return hipErrorInvalidValue;
         const int64_t ntm = (p.M + bm - 1) / bm;
         if (bn == 256) gsz = 16;
         const int64_t gmk = gsz / gn;

@@ -104,8 +104,6 @@ struct tmt_moe {
     float* pdwr = nullptr;
     uint16_t* pwu[kMaxExperts] = {};
     uint16_t* pwd[kMaxExperts] = {};
-    float* pdwu[kMaxExperts] = {};
-    float* pdwd[kMaxExperts] = {};
     int hn = 0;        // width of the first expert GEMM (h, or d for h == 0)
     int nblk_max = 0;  // router blocks at the largest T
     int device = 0;
@@ -287,7 +285,7 @@ Sizes plan(const tmt_moe_desc* user, tmt_moe* m) {
     // of 64 (transient: every call fills the ones it reads)
     const bool pad = is_padded(*user);
     size_t o_px = 0, o_py = 0, o_pdy = 0, o_pdx = 0, o_pwr = 0, o_pdwr = 0;
-    size_t o_pwu[kMaxExperts] = {}, o_pwd[kMaxExperts] = {}, o_pdwu[kMaxExperts] = {}, o_pdwd[kMaxExperts] = {};
+    size_t o_pwu[kMaxExperts] = {}, o_pwd[kMaxExperts] = {};
     if (pad) {
         o_px = W.add(T * D * 2);
         o_py = W.add(T * D * 2);
@@ -297,11 +295,7 @@ Sizes plan(const tmt_moe_desc* user, tmt_moe* m) {
         o_pdwr = W.add(E * D * 4);
         for (int64_t e = 0; e < E; ++e) {
             o_pwu[e] = W.add(hn * D * 2);
-            o_pdwu[e] = W.add(hn * D * 4);
-            if (h > 0) {
-                o_pwd[e] = W.add(D * h * 2);
-                o_pdwd[e] = W.add(D * h * 4);
-            }
+            if (h > 0) o_pwd[e] = W.add(D * h * 2);
         }
     }
     if (m) {
@@ -356,9 +350,7 @@ Sizes plan(const tmt_moe_desc* user, tmt_moe* m) {
             m->pdwr = (float*)(w + o_pdwr);
             for (int64_t e = 0; e < E; ++e) {
                 m->pwu[e] = (uint16_t*)(w + o_pwu[e]);
-                m->pdwu[e] = (float*)(w + o_pdwu[e]);
                 m->pwd[e] = h > 0 ? (uint16_t*)(w + o_pwd[e]) : nullptr;
-                m->pdwd[e] = h > 0 ? (float*)(w + o_pdwd[e]) : nullptr;
             }
         }
     }
@@ -659,7 +651,20 @@ struct LnGrad {
     float* dBeta;
 };
 
-// The backward's launches (arguments checked). With `ln`, dX is the gradient
+GemmParams dx_params(const tmt_moe* m, int T) {
+    GemmParams dx{};
+    dx.offsets = m->offsets; dx.order = m->order; dx.perm = m->perm; dx.E = m->desc.experts;
+    dx.N = m->desc.d; dx.K = m->hn; dx.slots = T * m->desc.topk;
+    return dx;
+}
+// Whether the backward's GEMM_DX runs over W_up transposed into the workspace.
+bool dx_transposed(const tmt_moe* m, int T) {
+    return T > 0 && m->wt != nullptr && gemm_tile(GEMM_DX, dx_params(m, T)).m == 256;
+}
+
+// The backward's launches (arguments checked). Wr and W_down have the
+// internal widths, and so has W_up unless dx_transposed; the weight gradients
+// are the caller's (dWr: internal width). With `ln`, dX is the gradient
 // at the LayerNorm output: for d <= kLnFusedMaxD the scatter consumes it in
 // registers (dX is not written), otherwise it lands in dX and the two-pass
 // LayerNorm backward follows.
@@ -669,6 +674,7 @@ int run_backward(tmt_moe* m, hipStream_t s, const uint16_t* dY, const uint16_t* 
                  float* const* dW_down, const LnGrad* ln) {
     const tmt_moe_desc& ds = m->desc;
     const int T = m->last_T, E = ds.experts, K = ds.topk, d = ds.d, h = ds.hidden, hn = m->hn;
+    const int hnu = h > 0 ? m->user.hidden : m->user.d;  // the caller's W_up is [hnu][user.d]
 
     if (T > 0) {
         CombineBwdParams cb{};
@@ -691,33 +697,33 @@ int run_backward(tmt_moe* m, hipStream_t s, const uint16_t* dY, const uint16_t* 
         }
         GemmParams dwd{};
         dwd.offsets = m->offsets; dwd.order = m->order; dwd.perm = m->perm; dwd.E = E;
-        dwd.M = d; dwd.N = h;
-        dwd.a = m->dO; dwd.lda = d; dwd.b = m->Aact; dwd.ldb = h; dwd.ldc = h;
+        dwd.M = d; dwd.N = h; dwd.m_out = m->user.d; dwd.n_out = m->user.hidden;
+        dwd.a = m->dO; dwd.lda = d; dwd.b = m->Aact; dwd.ldb = h; dwd.ldc = m->user.hidden;
         for (int e = 0; e < E; ++e) dwd.dw[e] = dW_down[e];
         LAUNCH(TMT_MOE_PH_GEMM_DW_DOWN, launch_gemm(GEMM_DW_DOWN, false, dwd, s));
     }
     GemmParams dwu{};
     dwu.offsets = m->offsets; dwu.order = m->order; dwu.perm = m->perm; dwu.E = E;
-    dwu.M = hn; dwu.N = d;
-    dwu.a = m->dU; dwu.lda = hn; dwu.b = m->Xg; dwu.ldb = d; dwu.ldc = d;
+    dwu.M = hn; dwu.N = d; dwu.m_out = hnu; dwu.n_out = m->user.d;
+    dwu.a = m->dU; dwu.lda = hn; dwu.b = m->Xg; dwu.ldb = d; dwu.ldc = m->user.d;
     for (int e = 0; e < E; ++e) dwu.dw[e] = dW_up[e];
     LAUNCH(TMT_MOE_PH_GEMM_DW_UP, launch_gemm(GEMM_DW_UP, false, dwu, s));
     if (T > 0) {
-        GemmParams dx{};
-        dx.offsets = m->offsets; dx.order = m->order; dx.perm = m->perm; dx.E = E;
-        dx.N = d; dx.K = hn; dx.slots = T * K;
+        GemmParams dx = dx_params(m, T);
         dx.a = m->dU; dx.lda = hn; dx.c = m->dXg; dx.ldc = d;
         for (int e = 0; e < E; ++e) dx.w[e] = W_up[e];
         dx.ldb = d;
         dx.part = m->split; dx.resident = m->resident;
-        if (m->wt != nullptr && gemm_tile(GEMM_DX, dx).m == 256) {
+        if (dx_transposed(m, T)) {
             // dXg = dU W_up as GEMM_DOWN over W_up^T: a transpose of the
             // weights (E * hn * d * 2 bytes each way) buys K-contiguous B
             // tiles for the GEMM (ds_read_b128 instead of the transposing
-            // 8-byte reads, half the LDS read instructions)
+            // 8-byte reads, half the LDS read instructions). It reads the
+            // caller's tensors (W_up holds them here) and pads as it goes.
             TransposeParams tp{};
             for (int e = 0; e < E; ++e) tp.src[e] = W_up[e];
-            tp.ld_src = d; tp.rows = hn; tp.cols = d; tp.dst = m->wt;
+            tp.ld_src = m->user.d; tp.rows_s = hnu; tp.cols_s = m->user.d;
+            tp.rows = hn; tp.cols = d; tp.dst = m->wt;
             LAUNCH(TMT_MOE_PH_GEMM_DX, launch_transpose_bf16(tp, E, s));
             GemmParams dt = dx;
             for (int e = 0; e < E; ++e) dt.w[e] = m->wt + (int64_t)e * d * hn;
@@ -842,7 +848,8 @@ int unpad_rows(const tmt_moe* m, hipStream_t s, int T, const uint16_t* src, uint
     void* b[1] = {dst};
     return copy_mats(s, a, b, 1, T, m->desc.d, T, m->user.d, 2);
 }
-// Router and expert weights into the handle's padded copies.
+// Router and expert weights into the handle's padded copies (W_up == nullptr:
+// the others only).
 int pad_weights(tmt_moe* m, hipStream_t s, const uint16_t* Wr, const uint16_t* const* W_up,
                 const uint16_t* const* W_down) {
     const int E = m->desc.experts, du = m->user.d, dp = m->desc.d, hu = m->user.hidden, hp = m->desc.hidden;
@@ -853,25 +860,19 @@ int pad_weights(tmt_moe* m, hipStream_t s, const uint16_t* Wr, const uint16_t* c
         void* b[1] = {m->pwr};
         if ((rc = copy_mats(s, a, b, 1, E, du, E, dp, 2))) return rc;
     }
-    if ((rc = copy_mats(s, (const void* const*)W_up, (void* const*)m->pwu, E, hnu, du, m->hn, dp, 2))) return rc;
+    if (W_up && (rc = copy_mats(s, (const void* const*)W_up, (void* const*)m->pwu, E, hnu, du, m->hn, dp, 2)))
+        return rc;
     if (hp > 0 && (rc = copy_mats(s, (const void* const*)W_down, (void* const*)m->pwd, E, du, hu, dp, hp, 2)))
         return rc;
     return TMT_MOE_OK;
 }
-// Gradients from the padded copies to the caller's (dWr may be NULL when E == 1).
-int unpad_grads(tmt_moe* m, hipStream_t s, float* dWr, float* const* dW_up, float* const* dW_down) {
-    const int E = m->desc.experts, du = m->user.d, dp = m->desc.d, hu = m->user.hidden, hp = m->desc.hidden;
-    const int hnu = hu > 0 ? hu : du;
-    int rc;
-    if (dWr) {
-        const void* a[1] = {m->pdwr};
-        void* b[1] = {dWr};
-        if ((rc = copy_mats(s, a, b, 1, E, dp, E, du, 4))) return rc;
-    }
-    if ((rc = copy_mats(s, (const void* const*)m->pdwu, (void* const*)dW_up, E, m->hn, dp, hnu, du, 4))) return rc;
-    if (hp > 0 && (rc = copy_mats(s, (const void* const*)m->pdwd, (void* const*)dW_down, E, dp, hp, du, hu, 4)))
-        return rc;
-    return TMT_MOE_OK;
+// The router gradient from the padded copy to the caller's (dWr may be NULL
+// when E == 1); the expert gradients are written in place.
+int unpad_dwr(tmt_moe* m, hipStream_t s, float* dWr) {
+    if (!dWr) return TMT_MOE_OK;
+    const void* a[1] = {m->pdwr};
+    void* b[1] = {dWr};
+    return copy_mats(s, a, b, 1, m->desc.experts, m->desc.d, m->desc.experts, m->user.d, 4);
 }
 
 }  // namespace
@@ -1144,14 +1145,16 @@ int tmt_moe_backward(tmt_moe* m, void* stream, const uint16_t* dY, const uint16_
     if (!m->padded)
         return run_backward(m, s, dY, X, Wr, W_up, W_down, aux_coef, z_coef, dX, dWr, dW_up, dW_down, nullptr);
     const int T = m->last_T;
-    if ((rc = pad_weights(m, s, Wr, W_up, W_down)) || (rc = pad_rows(m, s, T, X, m->px)) ||
+    // GEMM_DX over W_up transposed reads the caller's tensors
+    const bool wt = dx_transposed(m, T);
+    if ((rc = pad_weights(m, s, Wr, wt ? nullptr : W_up, W_down)) || (rc = pad_rows(m, s, T, X, m->px)) ||
         (rc = pad_rows(m, s, T, dY, m->pdy)))
         return rc;
-    if ((rc = run_backward(m, s, m->pdy, m->px, m->pwr, m->pwu, m->pwd, aux_coef, z_coef, m->pdx,
-                           dWr ? m->pdwr : nullptr, m->pdwu, m->pdwd, nullptr)))
+    if ((rc = run_backward(m, s, m->pdy, m->px, m->pwr, wt ? W_up : m->pwu, m->pwd, aux_coef, z_coef, m->pdx,
+                           dWr ? m->pdwr : nullptr, dW_up, dW_down, nullptr)))
         return rc;
     if ((rc = unpad_rows(m, s, T, m->pdx, dX))) return rc;
-    return unpad_grads(m, s, dWr, dW_up, dW_down);
+    return unpad_dwr(m, s, dWr);
 }
 
 int tmt_moe_backward_ln(tmt_moe* m, void* stream, const uint16_t* dY, const uint16_t* S,
@@ -1174,11 +1177,12 @@ int tmt_moe_backward_ln(tmt_moe* m, void* stream, const uint16_t* dY, const uint
     hipStream_t s = (hipStream_t)stream;
     if (!m->padded)
         return run_backward(m, s, dY, m->H, Wr, W_up, W_down, aux_coef, z_coef, m->dH, dWr, dW_up, dW_down, &lg);
-    if ((rc = pad_weights(m, s, Wr, W_up, W_down)) || (rc = pad_rows(m, s, T, dY, m->pdy))) return rc;
-    if ((rc = run_backward(m, s, m->pdy, m->H, m->pwr, m->pwu, m->pwd, aux_coef, z_coef, m->dH,
-                           dWr ? m->pdwr : nullptr, m->pdwu, m->pdwd, &lg)))
+    const bool wt = dx_transposed(m, T);
+    if ((rc = pad_weights(m, s, Wr, wt ? nullptr : W_up, W_down)) || (rc = pad_rows(m, s, T, dY, m->pdy))) return rc;
+    if ((rc = run_backward(m, s, m->pdy, m->H, m->pwr, wt ? W_up : m->pwu, m->pwd, aux_coef, z_coef, m->dH,
+                           dWr ? m->pdwr : nullptr, dW_up, dW_down, &lg)))
         return rc;
-    return unpad_grads(m, s, dWr, dW_up, dW_down);
+    return unpad_dwr(m, s, dWr);
 }
 
 int tmt_moe_read_stats(tmt_moe* m, void* stream, float* aux, float* z, int32_t* counts) {

@@ -124,6 +124,8 @@ struct GemmParams {
     int E;
     int M;                   // weight-gradient GEMMs: rows of C
     int N;                   // columns of C
+    int m_out, n_out;        // weight-gradient GEMMs: rows and columns of C that are stored (the
+                             // caller's widths; M and N are the operands', rounded up to 64)
     int K;                   // activation GEMMs: reduction length
     int slots;               // activation GEMMs: T*K routed rows (bounds the row tiles)
     const uint16_t* a; int64_t lda;   // activation operand
@@ -371,11 +373,13 @@ hipError_t launch_scatter(const ScatterParams& p, hipStream_t s);
 hipError_t launch_zero_f32(float* p, int64_t n, hipStream_t s);
 // out = bf16(in), round to nearest even.
 hipError_t launch_f32_to_bf16(const float* in, uint16_t* out, int64_t n, hipStream_t s);
-// dst + e * rows * cols = src[e]^T ([rows][cols] bf16, row stride ld_src ->
-// [cols][rows]); rows and cols multiples of 64.
+// dst + e * rows * cols = src[e]^T, zero-padded: src[e] is [rows_s][cols_s]
+// bf16 with row stride ld_src and any 2-byte alignment, the result
+// [cols][rows] with rows and cols multiples of 64 (rows_s <= rows, cols_s <= cols).
 struct TransposeParams {
     const uint16_t* src[kMaxExperts];
     int64_t ld_src;
+    int rows_s, cols_s;
     int rows, cols;
     uint16_t* dst;
 };

@@ -100,6 +100,18 @@ def test_width_matches_explicit_padding(T, d, E, K, h):
 
 
 @pytest.mark.parametrize("T,d,E,K,h", [
+    (6000, 700, 4, 2, 500),  # 256-row tiles: GEMM_DX over W_up transposed from the caller's tensors
+    (6001, 1285, 3, 2, 0),   # the same with reference experts and odd gradient rows (4-byte aligned stores)
+    (70, 3, 3, 2, 5),        # rows shorter than one 16-byte piece
+])
+def test_width_tiles_and_edges(orc, T, d, E, K, h):
+    """The padding copies, the transposed W_up and the cropped gradient
+    stores where rows cross 16-byte pieces, on both tile sizes."""
+    test_width_forward_backward(orc, T, d, E, K, h)
+    test_width_matches_explicit_padding(T, d, E, K, h)
+
+
+@pytest.mark.parametrize("T,d,E,K,h", [
     (14, 16, 2, 2, 0),
     (14, 16, 1, 1, 0),
     (1000, 32, 4, 2, 0),
