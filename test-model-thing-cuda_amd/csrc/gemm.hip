@@ -8,7 +8,8 @@
 //
 // Tile: 256 x 256 outputs per 256-thread workgroup (one workgroup per CU),
 // 4 waves in 2 x 2, each wave 128 x 128 = 4 x 4 v_mfma_f32_32x32x16_bf16
-// tiles (256 fp32 accumulators per lane, held in AGPRs).
+// tiles (256 fp32 accumulators per lane, held in AGPRs); 128 x 128 (64 x 64
+// per wave) where the large tiles would leave CUs idle (gemm_tile).
 //
 // Operand staging: direct global -> LDS loads (global_load_lds_dwordx4, the
 // data never passes through VGPRs). Two ring layouts:
@@ -19,9 +20,8 @@
 //     1 KiB load per 16 cycles when every row segment of the load is >= 128
 //     bytes, but only one per 29-34 cycles with 64-byte segments from L2 or
 //     HBM, so with K = 32 stages the loads alone filled the CU's load path;
-//   * one ring of NST stages of K = 32 (32 KiB for 256 x 256, 24 KiB for
-//     256 x 128), issued NST - 1 tiles ahead (weight-gradient GEMMs, the
-//     MXFP4 variants and 128-column tiles).
+//   * one ring of NST stages, issued NST - 1 tiles ahead (weight-gradient
+//     GEMMs and 128 x 128 tiles; see Ring).
 //   * K-contiguous operands (activations in every GEMM, weights in the
 //     forward) land as [256 rows][32] bf16, 16-byte chunks XOR-swizzled by
 //     (row >> 2) & 3, and are read with ds_read_b128.
@@ -41,6 +41,9 @@
 // row) so every global store is a 16-byte vector and each output row is
 // written as one contiguous 256-byte (bf16) or 512-byte (fp32) run; the
 // stores (and GEMM_DACT's pre-activation reads) are non-temporal.
+#include <algorithm>
+#include <cmath>
+
 #include "device_util.hpp"
 #include "moe_internal.hpp"
 
@@ -50,13 +53,8 @@ namespace {
 constexpr int BM = kGemmTileRows;  // tile rows of the large-problem kernels (TBM: the tile's own)
 
 // Tile geometry. BK_ is the K depth of one LDS stage (32 or 64), NST the
-// number of stages in the ring, BN_ the tile width and NWM_ the waves along
-// M (2 x NWM_ waves per workgroup):
-//   BN 256, NWM 2: one 4-wave workgroup per CU, 128 x 128 wave tiles;
-//   BN 256, NWM 4: one 8-wave workgroup per CU, 64 x 128 wave tiles (two
-//                  waves per SIMD on the same operand tiles);
-//   BN 128, NWM 2: two 4-wave workgroups per CU, 128 x 64 wave tiles, so one
-//                  workgroup's waits and epilogue overlap the other's MFMAs.
+// number of stages in the ring, BM_ x BN_ the tile and NWM_ the waves along
+// M (2 x NWM_ waves per workgroup).
 template <int BK_, int NST, int BN_, int NWM_ = 2, int BM_ = 256>
 struct Geo {
     static constexpr int BM = BM_;
@@ -76,7 +74,7 @@ struct Geo {
     static constexpr int DMA_PER_TILE = DMA_A + DMA_B;
     static constexpr int KC_ROWS = 1024 / (2 * BK);    // K-contiguous rows per wave load
     static constexpr int STEPS = BK / 16;              // MFMA k16 steps per stage
-    static constexpr int WGS = BN == 256 && BM == 256 ? 1 : 2;  // workgroups per CU
+    static constexpr int WGS = (BN == 256 && BM == 256) || (BK == 64 && NST > 2) ? 1 : 2;  // workgroups per CU
     // the epilogue's fp32 staging ([EPR][WTN] per wave); the kernel sizes the
     // ring (single or split) and checks the total
     static constexpr int EPI = NW * EPR * WTN * 4;
@@ -175,18 +173,31 @@ __device__ __forceinline__ void wait_vm() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N));
 }
 
+// Order of a launch's tiles. The hardware hands workgroup b to XCD b % 8, and
+// the list of (M tile, N tile) is dealt to the XCDs in pieces of consecutive
+// tiles, so that the tiles an XCD runs at a time are neighbours and its L2
+// serves each operand slice to several workgroups. The list goes by blocks of `rows` M
+// tiles, column by column inside a block, so that 32 (16) consecutive tiles
+// cover 4 x 8 (2 x 8) tiles where there are 8 columns or more.
+__device__ __forceinline__ void list_tile(int j, int mtiles, int ntn, int rows, int& mt, int& nt) {
+    const int blk = j / (rows * ntn), rem = j - blk * (rows * ntn);
+    const int in = min(rows, mtiles - blk * rows);  // the last block may be shorter
+    nt = rem / in;
+    mt = blk * rows + (rem - nt * in);
+}
+// M tiles per block of the activation GEMMs' list.
+__device__ __forceinline__ int list_rows(int ntn) { return ntn >= 8 ? 4 : 32 / ntn; }
+
 // Split-K of the last round (GEMM_DOWN / GEMM_DX, tiles 256 x BN, one
-// workgroup per CU). The activation tiles are numbered expert segment by
-// segment, M tile mt of all ntn column tiles; with ntn <= 8 and W resident
-// workgroups, the tiles with mt < cut (cut * ntn a multiple of W) fill whole
-// rounds. The R = (MT - cut) * ntn tiles left would otherwise run as one
-// short round on R CUs while the rest idle, so each is cut into S parts
-// along K (S = W / R, at least 8 k tiles a part). Part q of tail tile j is
-// workgroup F + j*S + q (F = cut * ntn, after the whole rounds in launch
-// order); it writes an fp32 partial tile, and split_fixup_kernel adds a
-// tile's S partials in part order and stores the bf16 result.
+// workgroup per CU). Of the launch's tiles, F (a multiple of the W resident
+// workgroups) fill whole rounds. The R tiles left would run as one short
+// round on R CUs while the rest idle, so each is cut into S parts along K
+// (S = W / R, at least 8 k tiles a part). Part q of tail tile j is workgroup
+// F + j*S + q, after the whole rounds in launch order; it writes an fp32
+// partial tile, and split_fixup_kernel adds a tile's S partials in part order
+// and stores the bf16 result.
 struct SplitPlan {
-    int cut = 0, F = 0, R = 0, S = 1, chunk = 0;  // chunk: reduction length of a part
+    int F = 0, R = 0, S = 1, chunk = 0;  // chunk: reduction length of a part
 };
 template <int TBM = BM>
 __device__ __forceinline__ int act_mtiles(const GemmParams& p) {
@@ -195,16 +206,12 @@ __device__ __forceinline__ int act_mtiles(const GemmParams& p) {
     return mt;
 }
 template <int BK>
-__device__ __forceinline__ SplitPlan split_plan(const GemmParams& p, int ntn, int mtiles) {
+__device__ __forceinline__ SplitPlan split_plan(const GemmParams& p, int tiles) {
     SplitPlan sp;
     const int W = p.resident;
-    // W a multiple of 256: the launch-order permutation of workgroups stays
-    // inside aligned blocks of 256, so the first F workgroups are the rounds' tiles.
-    if (p.part == nullptr || ntn > 8 || W <= 0 || W % 256 != 0 || W % ntn != 0) return sp;
-    const int per = W / ntn;  // M tiles per round
-    sp.cut = (mtiles / per) * per;
-    sp.F = sp.cut * ntn;
-    sp.R = (mtiles - sp.cut) * ntn;
+    if (p.part == nullptr || W <= 0 || W % 256 != 0) return sp;
+    sp.F = tiles / W * W;
+    sp.R = tiles - sp.F;
     const int nk = p.K / BK;
     int S = sp.R > 0 ? W / sp.R : 1;
     S = min(S, nk / 8);
@@ -308,17 +315,6 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
     const int ntn = (p.N + BN - 1) / BN;
 
     // ---- tile coordinates -------------------------------------------------
-    // The hardware hands workgroup b to XCD b % 8 and each XCD runs 32 at a
-    // time (one per CU). Workgroups b = 8j + x with j in [32t, 32t + 32) are
-    // therefore co-resident on XCD x; they get the 32 tiles of group
-    // G = 8t + x, laid out as gm x gn tiles (gn = min(tiles across N, 8)) so
-    // that the XCD's L2 serves each operand slice to several workgroups.
-    // Consecutive groups go to different XCDs, which spreads the long tiles
-    // of the weight-gradient GEMMs (experts in descending-count order).
-    const int lid = (((vb >> 8) << 3) + (vb & 7)) * 32 + ((vb >> 3) & 31);
-    const int G = lid >> 5, gi = lid & 31;
-    const int gn = min(ntn, 8), gm = 32 / gn;
-    const int ngn = (ntn + gn - 1) / gn;
     int e = -1, mt = 0, nt = 0;
     int row0 = 0, rows = 0;   // activation GEMMs: slot range of this tile
     int kbeg = 0, kend = 0;   // reduction range (slots for dW GEMMs)
@@ -328,37 +324,37 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
     if constexpr (!Tr::group_k) {
         kbeg = 0;
         kend = p.K;
+        const int tiles = et.total * ntn;
         SplitPlan sp;
         if constexpr (kSplitK) {
-            if (p.part != nullptr) sp = split_plan<BK>(p, ntn, et.total);
+            if (p.part != nullptr) sp = split_plan<BK>(p, tiles);
         }
-        if (p.xcd_runs) {
-            // Launches whose tiles all run at once: the tiles in (mt, nt)
-            // order, nt fastest, cut into 8 runs of `per`; workgroup vb runs
-            // on XCD vb % 8 and takes tile vb / 8 of that XCD's run. Every
-            // XCD gets the same number of tiles, and a run covers whole rows
-            // of tiles of one or two experts, whose weights its L2 keeps.
-            const int R = et.total * ntn;
-            const int per = (R + 7) / 8;
-            const int j = (vb & 7) * per + (vb >> 3);
-            if ((vb >> 3) >= per || j >= R) return;
-            mt = j / ntn;
-            nt = j - mt * ntn;
-        } else if (sp.S >= 2 && vb >= sp.F) {
+        int j;
+        if (sp.S >= 2 && vb >= sp.F) {
             const int u = vb - sp.F;
             if (u >= sp.R * sp.S) return;
-            const int j = u / sp.S, q = u - j * sp.S;
-            mt = sp.cut + j / ntn;
-            nt = j % ntn;
+            j = u / sp.S;
+            const int q = u - j * sp.S;
+            j += sp.F;
             kbeg = q * sp.chunk;
             kend = min(p.K, kbeg + sp.chunk);
             part_unit = u;
         } else {
-            if (gi >= gm * gn) return;
-            mt = (G / ngn) * gm + gi % gm;
-            nt = (G % ngn) * gn + gi / gm;
-            if (nt >= ntn) return;
+            // Whole rounds of 256: workgroups 8i + x with i in [32t, 32t + 32)
+            // are co-resident on XCD x and take 32 consecutive tiles; all
+            // XCDs are near each other in the list, so they also share the
+            // last-level cache. What is left of a round is cut into one run
+            // per XCD: every XCD gets the same number of tiles whatever the
+            // shape. (In fixed groups of 4 x 8 tiles, N = 2752's eleven
+            // columns gave every second XCD 12 tiles for the others' 32: UP
+            // and DACT at 15 K slots, K = 1024 took 150 and 138 us against
+            // 122 and 119.)
+            const int n = sp.S >= 2 ? sp.F : tiles, whole = n & ~255;
+            const int per = (n - whole + 7) / 8, i = (vb - whole) >> 3;
+            j = vb < whole ? (((vb >> 8) << 3) + (vb & 7)) * 32 + ((vb >> 3) & 31) : whole + (vb & 7) * per + i;
+            if (vb >= whole && (i >= per || j >= n)) return;
         }
+        list_tile(j, et.total, ntn, list_rows(ntn), mt, nt);
         if (!expert_tile<BM>(et, mt, e, row0, rows)) return;  // beyond the last tile of the last expert
         mlim = rows;
     } else {
@@ -373,18 +369,22 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
         //    and round, paired heaviest with lightest (XCD x runs groups
         //    16r + x and 16r + 15 - x). With 32-tile groups the XCD holding
         //    the heaviest expert's group could not be balanced.
+        // The list runs expert by expert (descending count), in groups of
+        // GSZ; a last round that is not full is cut into one run per XCD.
         constexpr int GSZ = BN == 256 ? 16 : 32;
         const int rnd = vb >> 8, xcd = vb & 7, sub = (vb >> 3) & 31;
         const int Gs = GSZ == 16 ? 16 * rnd + (sub < 16 ? xcd : 15 - xcd) : 8 * rnd + ((rnd & 1) ? 7 - xcd : xcd);
-        const int gk = sub & (GSZ - 1), gnk = min(ntn, 8), gmk = GSZ / gnk, ngnk = (ntn + gnk - 1) / gnk;
-        if (gk >= gmk * gnk) return;
         const int ntm = (p.M + BM - 1) / BM;
-        const int gpe = ((ntm + gmk - 1) / gmk) * ngnk;  // groups per expert
-        const int ei = Gs / gpe, g = Gs - ei * gpe;
-        if (ei >= p.E) return;
-        mt = (g / ngnk) * gmk + gk % gmk;
-        nt = (g % ngnk) * gnk + gk / gmk;
-        if (mt >= ntm || nt >= ntn) return;
+        const int n = p.E * ntm * ntn, rest = n - (vb & ~255);  // tiles from this round on
+        int j = Gs * GSZ + (sub & (GSZ - 1));
+        if (rest < 256) {
+            const int per = (rest + 7) / 8;
+            if (sub >= per) return;
+            j = (vb & ~255) + xcd * per + sub;
+        }
+        if (j >= n) return;
+        const int ei = j / (ntm * ntn);
+        list_tile(j - ei * (ntm * ntn), ntm, ntn, GSZ / min(ntn, 8), mt, nt);
         e = p.order[ei];
         kbeg = p.offsets[e];
         kend = p.offsets[e + 1];
@@ -884,17 +884,26 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
             // FLPR lanes per row (4 fp32 each), FRPI rows per instruction
             float* C = p.dw[e];
             const int cl = lane % FLPR;
+            const int n = nbase + cl * 4;
+            float* o0 = C + (int64_t)(mt * BM + mbase + pass * EPR) * p.ldc + col0 + n;
+            auto staged = [&](int rr) {
+                return *reinterpret_cast<const f32x4*>(stage_f + rr * WTN + ((cl ^ (rr & (CH - 1))) * 4));
+            };
+            // rows of any width: 16-byte stores at any float's address
+            if (mlim == BM && nlim == BN) {  // uniform: a whole tile
 #pragma unroll 4
-            for (int rr = lane / FLPR; rr < EPR; rr += FRPI) {
-                const int m = mbase + pass * EPR + rr;
-                const int n = nbase + cl * 4;
-                if (m >= mlim || n >= nlim) continue;
-                const f32x4 v = *reinterpret_cast<const f32x4*>(stage_f + rr * WTN + ((cl ^ (rr & (CH - 1))) * 4));
-                float* o = C + (int64_t)(mt * BM + m) * p.ldc + col0 + n;
-                // rows of any width: 16-byte stores at any float's address
-                if (n + 4 <= nlim) __builtin_nontemporal_store(v, reinterpret_cast<f32x4_any*>(o));
-                else
-                    for (int t = 0; t < nlim - n; ++t) o[t] = v[t];
+                for (int rr = lane / FLPR; rr < EPR; rr += FRPI)
+                    __builtin_nontemporal_store(staged(rr), reinterpret_cast<f32x4_any*>(o0 + (int64_t)rr * p.ldc));
+            } else {
+#pragma unroll 4
+                for (int rr = lane / FLPR; rr < EPR; rr += FRPI) {
+                    if (mbase + pass * EPR + rr >= mlim || n >= nlim) continue;
+                    const f32x4 v = staged(rr);
+                    float* o = o0 + (int64_t)rr * p.ldc;
+                    if (n + 4 <= nlim) __builtin_nontemporal_store(v, reinterpret_cast<f32x4_any*>(o));
+                    else
+                        for (int t = 0; t < nlim - n; ++t) o[t] = v[t];
+                }
             }
         }
         __syncthreads();
@@ -902,7 +911,7 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
 }
 
 template <int KIND, bool DUAL, int BK_, int NST, int BN_, int NWM_ = 2, int BM_ = 256>
-__global__ __launch_bounds__(128 * NWM_, (BN_ == 256 && BM_ == 256 ? 1 : 2)) void grouped_gemm_kernel(GemmParams p) {
+__global__ __launch_bounds__(128 * NWM_, (Geo<BK_, NST, BN_, NWM_, BM_>::WGS)) void grouped_gemm_kernel(GemmParams p) {
     __shared__ uint4 lds_raw[gemm_lds_bytes<KIND, BK_, NST, BN_, NWM_, BM_>() / 16];
     // the experts' tiles, once per workgroup (before any tile's stores, so
     // the vector load of the offsets waits on nothing else)
@@ -921,8 +930,8 @@ __global__ __launch_bounds__(128 * NWM_, (BN_ == 256 && BM_ == 256 ? 1 : 2)) voi
 // thread t adds 8 columns of one row.
 template <int BK, int BN>
 __global__ __launch_bounds__(256) void split_fixup_kernel(GemmParams p) {
-    const int ntn = (p.N + BN - 1) / BN;
-    const SplitPlan sp = split_plan<BK>(p, ntn, act_mtiles(p));
+    const int ntn = (p.N + BN - 1) / BN, mtiles = act_mtiles(p);
+    const SplitPlan sp = split_plan<BK>(p, mtiles * ntn);
     if (sp.S < 2) return;
     constexpr int kSlabs = BM / 8;
     const int tid = threadIdx.x;
@@ -930,8 +939,8 @@ __global__ __launch_bounds__(256) void split_fixup_kernel(GemmParams p) {
     uint16_t* C = reinterpret_cast<uint16_t*>(p.c);
     for (int w = blockIdx.x; w < sp.R * kSlabs; w += gridDim.x) {
         const int j = w / kSlabs, slab = w % kSlabs;
-        const int mt = sp.cut + j / ntn, nt = j % ntn;
-        int e, row0 = 0, rows = 0;
+        int mt, nt, e, row0 = 0, rows = 0;
+        list_tile(sp.F + j, mtiles, ntn, list_rows(ntn), mt, nt);
         act_tile(p, mt, e, row0, rows);
         const int row = slab * 8 + rr;
         if (e < 0 || row >= rows || nt * BN + col >= p.N) continue;
@@ -960,148 +969,152 @@ __global__ __launch_bounds__(256) void split_fixup_kernel(GemmParams p) {
 
 }  // namespace
 
-// Tile depth and ring per kind and tile width: split rings of K = 64 for the
-// activation GEMMs on 256 columns; K = 32 rings otherwise (4 stages of 32 KiB
-// at 256 columns, 3 of 24 KiB at 128 columns with two workgroups per CU).
-// 128 x 128 tiles (two workgroups per CU, 64 KiB each, the size of the
-// epilogue's staging anyway): 4 stages of K = 32, or with K64 2 stages of
-// K = 64, whose 128-byte row segments the CU's load path takes at twice the
-// rate of 64-byte ones (reference profile shape, K = 1280: up GEMM 25
-// against 30 us; at K = 256 the deeper K = 32 ring is as fast or faster).
-template <int KIND, int BN, int TBM = BM, bool K64 = false>
+// Ring of a kind and tile size:
+//   256 x 256 (one workgroup per CU): split rings of K = 64 (activation
+//   GEMMs), 4 stages of K = 32 (weight gradients);
+//   128 x 128 activation tiles: 2 stages of K = 64, two workgroups per CU
+//   (64 KiB each, the size of the epilogue's staging anyway), or DEEP, 4
+//   stages, one workgroup per CU. With two stages a lone workgroup waits out
+//   a memory round trip per K = 64 step (about 1.1 us); with four it is down
+//   to 0.72 us, mostly its LDS reads. K = 64 makes 128-byte row segments,
+//   which the CU's load path takes at twice the rate of 64-byte ones;
+//   128 x 128 weight-gradient tiles: 4 stages of K = 32, two workgroups per CU.
+template <int KIND, int TBM = BM, bool DEEP = false>
 struct Ring {
-    static constexpr bool split = split_ring<KIND, 64, BN, 2, TBM>();
-    static constexpr bool k64 = K64 && TBM == 128;
+    static constexpr bool split = split_ring<KIND, 64, TBM, 2, TBM>();
+    static constexpr bool k64 = TBM == 128 && !Traits<KIND>::group_k;
     static constexpr int BK = split || k64 ? 64 : 32;
-    static constexpr int NST = split ? 3 : k64 ? 2 : (BN == 256 || TBM == 128 ? 4 : 3);
+    static constexpr int NST = split ? 3 : k64 && !DEEP ? 2 : 4;
 };
 
 // grid: the launch-order blocks of the tile map. Persistent kinds run
 // min(grid, CUs rounded down to a multiple of 8) workgroups over them.
-template <int KIND, bool DUAL, int BN, int NWM = 2, int TBM = BM, bool K64 = false>
+template <int KIND, bool DUAL, int TBM = BM, bool DEEP = false>
 hipError_t launch_kind(const GemmParams& p, unsigned grid, hipStream_t s) {
-    using R = Ring<KIND, BN, TBM, K64>;
+    using R = Ring<KIND, TBM, DEEP>;
     GemmParams q = p;
     q.vblocks = (int)grid;
     unsigned g = grid;
-    if constexpr (persistent_tiles<KIND, R::BK, BN, NWM, TBM>()) {
+    if constexpr (persistent_tiles<KIND, R::BK, TBM, 2, TBM>()) {
         const unsigned cus = (unsigned)(cu_count() / 8 * 8);
         if (cus >= 8 && g > cus) g = cus;
     }
-    grouped_gemm_kernel<KIND, DUAL, R::BK, R::NST, BN, NWM, TBM><<<g, 128 * NWM, 0, s>>>(q);
+    grouped_gemm_kernel<KIND, DUAL, R::BK, R::NST, TBM, 2, TBM><<<g, 256, 0, s>>>(q);
     return hipGetLastError();
 }
 
-// Tile width per GEMM kind (BN 128 = two workgroups per CU). Measured in the
-// c3 step: every GEMM runs fastest on 256-column tiles (UP, DOWN, DX and DACT
-// on split rings; UP 1.26 against 1.29 ms with two 128-column workgroups per
-// CU). DACT moved to 256 columns once its epilogue no longer evaluated
-// silu'(U) itself (1.22 against 1.24 ms, and the weight-gradient GEMMs after
-// it 0.02-0.04 ms faster); while it did, the co-resident second workgroup of
-// the 128-column tiles covered that VALU work and won. The weight-gradient
-// GEMMs run 256-column tiles in balanced 16-tile groups (4-6% faster than two
-// 128-column workgroups).
-// Small problems: a launch whose 256 x 256 tiles would leave most CUs idle
-// runs 128 x 128 tiles (four times the tiles, two workgroups per CU). At
-// the reference's profile shape (4096 slots, d = 1280, h = 0) the up GEMM
-// took 30 us on 128 x 128 tiles against 29 us on 256 x 128 and 35 us on
-// 256 x 256 (all with the XCD runs of launch_gemm_tile); at TMT's default
-// width (2048 slots, d = 256) 9 against 12 and 16 us.
-static int64_t tiles_256(GemmKind kind, const GemmParams& p) {
-    const int64_t ntn = (p.N + 255) / 256;
-    if (kind == GEMM_DW_DOWN || kind == GEMM_DW_UP) return (int64_t)p.E * ((p.M + BM - 1) / BM) * ntn;
-    return ((int64_t)p.slots + BM - 1) / BM * ntn;  // lower bound (experts' partial tiles aside)
+// Tiles of `rows` rows that the experts' segments make at even routing: one
+// per expert while the mean is well below `rows`; above, half of each
+// expert's last tile is empty on average, or, with few tiles per expert, the
+// mean's own last tile where it lies clear of a multiple of `rows`.
+static double act_tiles(const GemmParams& p, int rows) {
+    const double used = std::min(p.E, p.slots), m = p.slots / (used > 0 ? used : 1.0) / rows;
+    return used * (m <= 0.85 ? 1.0 : m < 3.0 ? std::min(m + 0.5, std::ceil(m + 0.15)) : m + 0.5);
+}
+// Estimated time (us) of an activation GEMM on each tile, from what the
+// kernels measured on one MI355X over K = 256 .. 4096 and 0.2 .. 33 rounds
+// (nk: K = 64 steps):
+//   256 x 256, a round of one tile per CU: 17 + 1.24 nk where the epilogue
+//     evaluates or multiplies by the SiLU terms (GEMM_UP with hidden > 0,
+//     GEMM_DACT), else 9 + 1.56 nk; GEMM_DOWN and GEMM_DX split the last
+//     round along K, which costs the partial tiles' write and fix-up (up to
+//     28 us when it fills the chip);
+//   128 x 128, a round of two per CU: 5 + 1.1 nk (full or not);
+//   128 x 128 deep, one per CU: 4 + 0.72 nk, better than two per CU only
+//     while every tile has a CU of its own.
+// Small problems leave CUs idle or end in a nearly empty round on the large
+// tiles. Measured (us; 256 x 256 / 128 x 128 / deep): 777 tokens on 16
+// experts, top-4, N = 1024, K = 4096 70 / 77 / 52; 4096 slots, E = 8,
+// N = K = 1280 35 / 25 / 30; 8192 slots, E = 8, N = 2048, K = 768 61 / 55 /
+// 61; 32768 slots, E = 8, N = 2048, K = 512 146 / 133 / 164; 131072 slots,
+// E = 16, N = 4096, K = 1024 1228 / 1456 / -.
+static GemmTile act_tile_choice(GemmKind kind, const GemmParams& p) {
+    const double cus = cu_count(), nk = p.K / 64.0;
+    const bool silu = kind == GEMM_DACT || (kind == GEMM_UP && p.c2 != nullptr);
+    const double t256 = act_tiles(p, 256) * ((p.N + 255) / 256), t128 = act_tiles(p, 128) * ((p.N + 127) / 128);
+    const double round256 = silu ? 17.0 + 1.24 * nk : 9.0 + 1.56 * nk;
+    double c256 = std::ceil(t256 / cus) * round256;
+    if ((kind == GEMM_DOWN || kind == GEMM_DX) && p.part != nullptr) {
+        const double whole = std::floor(t256 / cus), rest = std::ceil(t256 - whole * cus);
+        const double parts = rest > 0 ? std::min(std::floor(cus / rest), std::floor(nk / 8)) : 1.0;
+        if (parts >= 2) c256 = whole * round256 + 12.0 + 1.56 * nk / parts + 28.0 * rest * parts / cus;
+    }
+    const double c128 = std::ceil(t128 / (2 * cus)) * (5.0 + 1.1 * nk);
+    const double cdeep = std::ceil(t128 / cus) * (4.0 + 0.72 * nk);
+    if (c256 <= c128 && c256 <= cdeep) return GemmTile{256};
+    return GemmTile{128, t128 <= cus && cdeep < c128};
 }
 
 GemmTile gemm_tile(GemmKind kind, const GemmParams& p) {
-    if (kind == GEMM_UP_FP4 || kind == GEMM_DOWN_FP4) return GemmTile{256, 256};
-    if (2 * tiles_256(kind, p) < cu_count()) {
-        const bool group_k = kind == GEMM_DW_DOWN || kind == GEMM_DW_UP;
-        return GemmTile{128, 128, !group_k && p.K % 64 == 0 && p.K >= 512};
+    if (kind == GEMM_UP_FP4 || kind == GEMM_DOWN_FP4) return GemmTile{256};
+    if (kind == GEMM_DW_DOWN || kind == GEMM_DW_UP) {
+        // Weight gradients: 128 x 128 tiles (two per CU) where the 256 x 256
+        // ones fill at most half of the CUs. d = 512, h = 2048, E = 8 (128
+        // large tiles): 113 -> 86 us each at 32768 slots; d = h = 1280, E = 8
+        // (200 large tiles): 28 us on large, 30 on small ones.
+        const int64_t tiles = (int64_t)p.E * ((p.M + 255) / 256) * ((p.N + 255) / 256);
+        return GemmTile{2 * tiles <= cu_count() ? 128 : 256};
     }
-    return GemmTile{256, 256};
+    return act_tile_choice(kind, p);
 }
 
 hipError_t launch_gemm_tile(GemmKind kind, bool dual, const GemmParams& p, GemmTile tile, hipStream_t s) {
-    const int bn = tile.n, bm = tile.m;
+    const int bn = tile.m, bm = tile.m;
     if (p.N % 8 != 0 || p.N <= 0) return hipErrorInvalidValue;
-    if (bn != 256 && bn != 128) return hipErrorInvalidValue;
-    if (bm != 256 && !(bm == 128 && bn == 128)) return hipErrorInvalidValue;
-    if (tile.k64 && (bm != 128 || p.K % 64 != 0 || kind == GEMM_DW_DOWN || kind == GEMM_DW_UP))
-        return hipErrorInvalidValue;
+    if (bm != 256 && bm != 128) return hipErrorInvalidValue;
     const bool group_k = kind == GEMM_DW_DOWN || kind == GEMM_DW_UP;
     const bool fp4 = kind == GEMM_UP_FP4 || kind == GEMM_DOWN_FP4;
-    if (fp4 && (p.K % 64 != 0 || bn != 256 || bm != 256)) return hipErrorInvalidValue;
+    if (tile.deep && (bm != 128 || group_k)) return hipErrorInvalidValue;
+    if (fp4 && bm != 256) return hipErrorInvalidValue;
     const int64_t ntn = (p.N + bn - 1) / bn;
-    const int64_t gn = ntn < 8 ? ntn : 8, gm = 32 / gn;
-    const int64_t ngn = (ntn + gn - 1) / gn;
-    int64_t groups;
-    int64_t gsz = 32;  // tiles per group (weight-gradient GEMMs on 256 columns: 16)
+    int64_t grid;
     if (group_k) {
         if (p.M % 8 != 0 || p.M <= 0) return hipErrorInvalidValue;
         if (p.m_out > p.M || p.n_out > p.N || p.M - p.m_out >= 64 || p.N - p.n_out >= 64 || p.ldc < p.n_out)
             return hipErrorInvalidValue;
-        const int64_t ntm = (p.M + bm - 1) / bm;
-        if (bn == 256) gsz = 16;
-        const int64_t gmk = gsz / gn;
-        groups = (int64_t)p.E * ((ntm + gmk - 1) / gmk) * ngn;
+        // whole rounds of 8 XCDs x 32 workgroups keep the block -> tile map a bijection
+        grid = ((int64_t)p.E * ((p.M + bm - 1) / bm) * ntn + 255) / 256 * 256;
     } else {
-        if (p.K % (bn == 256 && !fp4 ? 64 : 32) != 0) return hipErrorInvalidValue;
+        if (p.K % 64 != 0) return hipErrorInvalidValue;
         // sum_e ceil(cnt_e / bm) <= ceil(slots / bm) + E - 1
-        const int64_t mtiles = (int64_t)(p.slots + bm - 1) / bm + p.E;
-        groups = ((mtiles + gm - 1) / gm) * ngn;
+        const int64_t tiles = ((int64_t)(p.slots + bm - 1) / bm + p.E) * ntn;
+        grid = (tiles + 7) / 8 * 8;  // eight equal runs
     }
-    // whole rounds of 8 XCDs x 32 workgroups keep the block -> tile map a bijection
-    int64_t grid = (groups * gsz + 255) / 256 * 256;
-    GemmParams q = p;
-    q.xcd_runs = 0;
-    if (!group_k && !fp4) {
-        // every tile resident at once (two workgroups per CU below 256 x 256):
-        // 8 equal runs of tiles, one per XCD (at most 8 * ceil(tiles / 8) blocks)
-        const int64_t mt_max = (int64_t)(p.slots + bm - 1) / bm + p.E;
-        const int64_t tiles = mt_max * ntn;
-        const int64_t slots_resident = (int64_t)cu_count() * (bn == 256 && bm == 256 ? 1 : 2);
-        if (tiles <= slots_resident) {
-            q.xcd_runs = 1;
-            grid = (tiles + 7) / 8 * 8;
-        }
-    }
+    const GemmParams& q = p;
     // split-K tail (GEMM_DOWN / GEMM_DX on 256-column tiles): its parts are
     // the workgroups after the whole rounds, at most `resident` of them.
-    const bool split = (kind == GEMM_DOWN || kind == GEMM_DX) && bn == 256 && bm == 256 && p.part != nullptr && !q.xcd_runs &&
+    const bool split = (kind == GEMM_DOWN || kind == GEMM_DX) && bm == 256 && p.part != nullptr &&
                        p.resident > 0 && p.resident % 256 == 0;
     if (split) grid += p.resident;
     if (grid <= 0) return hipSuccess;
     if (grid > 0x7fffffff) return hipErrorInvalidValue;
     const unsigned g = (unsigned)grid;
-#define TMT_BN(KIND_, DUAL_)                                      \
-    (bn == 256     ? launch_kind<KIND_, DUAL_, 256>(q, g, s)      \
-     : bm == 256   ? launch_kind<KIND_, DUAL_, 128>(q, g, s)      \
-     : !tile.k64   ? launch_kind<KIND_, DUAL_, 128, 2, 128>(q, g, s) \
-                   : launch_kind<KIND_, DUAL_, 128, 2, 128, true>(q, g, s))
     if (split) {
-        // bn == 256 here, so launch_kind runs the 256-column kernel
-        hipError_t err = kind == GEMM_DOWN ? launch_kind<GEMM_DOWN, false, 256>(q, g, s)
-                                           : launch_kind<GEMM_DX, false, 256>(q, g, s);
+        hipError_t err = kind == GEMM_DOWN ? launch_kind<GEMM_DOWN, false>(q, g, s) : launch_kind<GEMM_DX, false>(q, g, s);
         if (err != hipSuccess) return err;
-        static_assert(Ring<GEMM_DOWN, 256>::BK == Ring<GEMM_DX, 256>::BK, "one split plan for DOWN and DX");
+        static_assert(Ring<GEMM_DOWN>::BK == Ring<GEMM_DX>::BK, "one split plan for DOWN and DX");
         // 4 workgroups per CU: the (tile, 8-row slab) items are short and latency-bound
-        split_fixup_kernel<Ring<GEMM_DOWN, 256>::BK, 256><<<p.resident * 4, 256, 0, s>>>(q);
+        split_fixup_kernel<Ring<GEMM_DOWN>::BK, 256><<<p.resident * 4, 256, 0, s>>>(q);
         return hipGetLastError();
     }
+#define TMT_ACT(KIND_, DUAL_)                                   \
+    (bm == 256    ? launch_kind<KIND_, DUAL_>(q, g, s)          \
+     : !tile.deep ? launch_kind<KIND_, DUAL_, 128>(q, g, s)     \
+                  : launch_kind<KIND_, DUAL_, 128, true>(q, g, s))
+#define TMT_DW(KIND_) (bm == 256 ? launch_kind<KIND_, false>(q, g, s) : launch_kind<KIND_, false, 128>(q, g, s))
     switch (kind) {
-        case GEMM_UP: return dual ? TMT_BN(GEMM_UP, true) : TMT_BN(GEMM_UP, false);
-        case GEMM_DOWN: return TMT_BN(GEMM_DOWN, false);
-        case GEMM_DACT: return TMT_BN(GEMM_DACT, false);
-        case GEMM_DX: return TMT_BN(GEMM_DX, false);
-        case GEMM_DW_DOWN: return TMT_BN(GEMM_DW_DOWN, false);
-        case GEMM_DW_UP: return TMT_BN(GEMM_DW_UP, false);
-        case GEMM_UP_FP4:
-            return dual ? launch_kind<GEMM_UP_FP4, true, 256>(q, g, s) : launch_kind<GEMM_UP_FP4, false, 256>(q, g, s);
-        case GEMM_DOWN_FP4: return launch_kind<GEMM_DOWN_FP4, false, 256>(q, g, s);
+        case GEMM_UP: return dual ? TMT_ACT(GEMM_UP, true) : TMT_ACT(GEMM_UP, false);
+        case GEMM_DOWN: return TMT_ACT(GEMM_DOWN, false);
+        case GEMM_DACT: return TMT_ACT(GEMM_DACT, false);
+        case GEMM_DX: return TMT_ACT(GEMM_DX, false);
+        case GEMM_DW_DOWN: return TMT_DW(GEMM_DW_DOWN);
+        case GEMM_DW_UP: return TMT_DW(GEMM_DW_UP);
+        case GEMM_UP_FP4: return dual ? launch_kind<GEMM_UP_FP4, true>(q, g, s) : launch_kind<GEMM_UP_FP4, false>(q, g, s);
+        case GEMM_DOWN_FP4: return launch_kind<GEMM_DOWN_FP4, false>(q, g, s);
         default: return hipErrorInvalidValue;
     }
-#undef TMT_BN
+#undef TMT_ACT
+#undef TMT_DW
 }
 
 hipError_t launch_gemm(GemmKind kind, bool dual, const GemmParams& p, hipStream_t s) {

@@ -152,9 +152,6 @@ struct GemmParams {
     // Set by the launcher: launch-order blocks of the tile map (persistent
     // grouped GEMMs loop over them).
     int vblocks;
-    // Set by the launcher for activation GEMMs whose tiles all run at once:
-    // the (M tile, N tile) list is cut into 8 equal runs, one per XCD.
-    int xcd_runs;
 };
 hipError_t launch_gemm(GemmKind kind, bool dual, const GemmParams& p, hipStream_t s);
 // Rows of an activation-GEMM tile, and the fp32 partial buffer the split-K
@@ -162,11 +159,12 @@ hipError_t launch_gemm(GemmKind kind, bool dual, const GemmParams& p, hipStream_
 constexpr int kGemmTileRows = 256;
 inline size_t gemm_split_floats(int resident) { return (size_t)resident * kGemmTileRows * 256; }
 int cu_count();  // compute units of the current device (cached per device)
-// Same with an explicit tile shape: 256 x 256 (one workgroup per CU),
-// 256 x 128 or 128 x 128 (two workgroups per CU; bf16 kinds only).
+// Same with an explicit tile: m x m outputs, 256 (one workgroup per CU) or 128
+// (two per CU; deep, activation GEMMs only: one per CU, a ring of twice the
+// stages). MXFP4 kinds: 256.
 struct GemmTile {
-    int m, n;
-    bool k64 = false;  // 128 x 128 tiles: 2 stages of K = 64 instead of 4 of K = 32
+    int m;
+    bool deep = false;
 };
 GemmTile gemm_tile(GemmKind kind, const GemmParams& p);  // the shape launch_gemm picks
 hipError_t launch_gemm_tile(GemmKind kind, bool dual, const GemmParams& p, GemmTile tile, hipStream_t s);
@@ -401,6 +399,7 @@ struct LayerNormParams {
     float* partial;          // [ln_chunks(T)][2][ln_width4(d)] dgamma / dbeta chunk sums
     float* dgamma;           // [d]
     float* dbeta;            // [d]
+    bool reread = false;     // forward: the next kernel reads H (no non-temporal stores)
 };
 int ln_chunks(int T);
 // Row stride of the dgamma / dbeta partials: d rounded up to a multiple of 4.

@@ -186,6 +186,26 @@ def test_shapes_against_oracle(orc, T, d, E, K, h):
 
 
 @pytest.mark.parametrize("T,d,E,K,h", [
+    (700, 1088, 3, 2, 1344),   # 128-row tiles with the deep ring: 17 and 21 K steps over its four stages
+    (1000, 512, 2, 2, 4096),   # DOWN and DX on fewer large tiles than CUs, every one split along K
+    (4000, 640, 2, 2, 2752),   # 22 column tiles of 128: short last block and last run of the tile list
+    (6000, 1024, 2, 2, 2752),  # 11 column tiles of 256: whole rounds, then one run per XCD
+    (3000, 1280, 8, 2, 0),     # five column tiles; weight gradients in a round that is not full
+])
+def test_tile_lists_and_rings(orc, T, d, E, K, h):
+    """Every tile size of the grouped GEMMs where its tile list or its ring
+    has an edge, forward and backward against the oracle, with the bounds of
+    the parity tests above."""
+    say(f"tile lists T={T} d={d} E={E} K={K} h={h} fwd+bwd")
+    case = make_case(T, d, E, K, h, seed=T + d)
+    g = run_gpu(case, K, h, backward=True, aux=0.1, z=1e-3)
+    r = oracle_case(orc, case, K, h, backward=True, aux=0.1, z=1e-3)
+    check_routing(g, r, E)
+    assert rel_l2(g["Y"], r["Y"]) <= REL_L2
+    check_grads(g, r, h, E)
+
+
+@pytest.mark.parametrize("T,d,E,K,h", [
     (4, 1024, 16, 1, 256),     # fewer picks than experts: most of the expert-indexed grid is empty
     (16, 1024, 64, 2, 256),    # 64 experts: dispatch tables over every lane of the wave
     (33, 1024, 8, 2, 512),     # four 16-row blocks per expert
