@@ -343,16 +343,19 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
             // Whole rounds of 256: workgroups 8i + x with i in [32t, 32t + 32)
             // are co-resident on XCD x and take 32 consecutive tiles; all
             // XCDs are near each other in the list, so they also share the
-            // last-level cache. What is left of a round is cut into one run
-            // per XCD: every XCD gets the same number of tiles whatever the
-            // shape. (In fixed groups of 4 x 8 tiles, N = 2752's eleven
+            // last-level cache. Where few rounds run, what is left of the last
+            // one is cut into one run per XCD, so that every XCD gets the same
+            // number of tiles (eleven columns, 715 tiles: UP 121.3 us, dealt
+            // as another round 122.6; after 32 rounds the deal keeps the
+            // neighbours together: UP at 8304 tiles 1244 against 1248 us).
+            // (In fixed groups of 4 x 8 tiles, N = 2752's eleven
             // columns gave every second XCD 12 tiles for the others' 32: UP
             // and DACT at 15 K slots, K = 1024 took 150 and 138 us against
             // 122 and 119.)
-            const int n = sp.S >= 2 ? sp.F : tiles, whole = n & ~255;
+            const int n = sp.S >= 2 ? sp.F : tiles, whole = n >= 8 * 256 ? (n + 255) & ~255 : n & ~255;
             const int per = (n - whole + 7) / 8, i = (vb - whole) >> 3;
             j = vb < whole ? (((vb >> 8) << 3) + (vb & 7)) * 32 + ((vb >> 3) & 31) : whole + (vb & 7) * per + i;
-            if (vb >= whole && (i >= per || j >= n)) return;
+            if (j >= n || (vb >= whole && i >= per)) return;
         }
         list_tile(j, et.total, ntn, list_rows(ntn), mt, nt);
         if (!expert_tile<BM>(et, mt, e, row0, rows)) return;  // beyond the last tile of the last expert
@@ -1078,7 +1081,7 @@ hipError_t launch_gemm_tile(GemmKind kind, bool dual, const GemmParams& p, GemmT
         if (p.K % 64 != 0) return hipErrorInvalidValue;
         // sum_e ceil(cnt_e / bm) <= ceil(slots / bm) + E - 1
         const int64_t tiles = ((int64_t)(p.slots + bm - 1) / bm + p.E) * ntn;
-        grid = (tiles + 7) / 8 * 8;  // eight equal runs
+        grid = tiles >= 8 * 256 ? (tiles + 255) / 256 * 256 : (tiles + 7) / 8 * 8;  // whole rounds, or eight equal runs
     }
     const GemmParams& q = p;
     // split-K tail (GEMM_DOWN / GEMM_DX on 256-column tiles): its parts are

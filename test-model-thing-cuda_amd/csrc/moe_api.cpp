@@ -493,8 +493,8 @@ int route(tmt_moe* m, hipStream_t s, int T, const uint16_t* X, const uint16_t* W
     PermuteParams pp{};
     pp.idx = m->idx; pp.blkbase = m->blkbase; pp.T = T; pp.E = E; pp.K = K;
     pp.rows_per_block = rpb; pp.perm = m->perm; pp.slot_of = m->slot_of;
-    if (nblk > 0 && nblk <= kFusedScanBlocks) {
-        // few router blocks: the permutation kernel does the scan itself
+    if (permute_scan_fits(nblk, E)) {
+        // not too many router blocks: the permutation kernel does the scan itself
         LAUNCH(TMT_MOE_PH_PERMUTE, launch_permute_scan(pp, sp, nblk, s));
         return TMT_MOE_OK;
     }

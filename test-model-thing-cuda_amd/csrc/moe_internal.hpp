@@ -82,9 +82,8 @@ struct PermuteParams {
     int32_t* slot_of;        // [T][K] (token, j) -> slot
 };
 hipError_t launch_permute(const PermuteParams& p, int nblk, hipStream_t s);
-// scan + permute in one launch for nblk <= kFusedScanBlocks router blocks
-// (blkbase is not written).
-constexpr int kFusedScanBlocks = 64;
+// scan + permute in one launch where permute_scan_fits (blkbase is not written).
+bool permute_scan_fits(int nblk, int E);
 hipError_t launch_permute_scan(const PermuteParams& p, const ScanParams& sp, int nblk, hipStream_t s);
 
 // T <= kSmallRouteTokens: router + scan + permute in one launch, one block

@@ -948,9 +948,11 @@ __global__ __launch_bounds__(1024) void scan_kernel(ScanParams p) {
     const int tid = threadIdx.x;
     const int E = p.E, nblk = p.nblk;
 
-    // 1) per (segment, expert) sums of the block histograms (no more
-    // segments than blocks: the serial scans of step 2 walk every segment)
-    const int S = max(1, min(1024 / E, nblk));
+    // 1) per (segment, expert) sums of the block histograms (few segments:
+    // the serial scans of step 2 walk every one; E = 8 and 256 blocks took
+    // 11 us with two blocks per segment),
+    // and a segment is at least one batch of 8 loads
+    const int S = max(1, min(1024 / E, (nblk + 7) / 8));
     const int chunk = (nblk + S - 1) / S;
     // (Loads in batches of 8 at clamped addresses, added in ascending order:
     // one memory round trip per batch instead of one per block.)
@@ -969,7 +971,7 @@ __global__ __launch_bounds__(1024) void scan_kernel(ScanParams p) {
     }
     // 1b) per (segment, statistic) sums of the block statistics
     const int E1 = E + 1;
-    const int S2 = max(1, min(1024 / E1, nblk));
+    const int S2 = max(1, min(1024 / E1, (nblk + 7) / 8));
     const int chunk2 = (nblk + S2 - 1) / S2;
     if (tid < S2 * E1) {
         const int q = tid % E1, seg = tid / E1;
@@ -1100,48 +1102,77 @@ __global__ __launch_bounds__(kThreads) void permute_kernel(PermuteParams p) {
     }
 }
 
-// The permutation with the scan folded in, for grids of at most
-// kFusedScanBlocks router blocks: every block adds the block histograms
-// itself (the totals, and the counts of the blocks before it, in ascending
-// block order) to find its own bases, and block 0 writes the counts,
-// offsets, order and statistics (block statistics added in ascending block
-// order). One launch fewer where the scan's single workgroup was mostly
-// launch latency. Slots are the same as scan_kernel + permute_kernel give.
-__global__ __launch_bounds__(kThreads) void permute_scan_kernel(PermuteParams p, ScanParams sp) {
+// The permutation with the scan folded in (permute_scan_fits): every block
+// adds the block histograms itself (the totals, and the counts of the blocks
+// before it) to find its own bases, and block 0 writes the counts, offsets,
+// order and statistics. The router blocks are cut into one segment per group
+// of threads (thread t: expert t % ep of segment t / ep), whose loads go out
+// eight at a time; segments are added in ascending order, so the statistics
+// are run-to-run deterministic. One launch fewer, and the sums of up to 256
+// blocks cost each permutation block about what the scan's single workgroup
+// took for its first pass. Slots are the same as scan_kernel + permute_kernel
+// give. Scan and permutation (event-timed, us): T = 16384, E = 8, 256 router
+// blocks 20.0 -> 8.5; T = 32768, E = 16, 256 blocks 21.2 -> 13.6; T = 14283,
+// E = 4, 224 blocks 25.3 -> 8.4.
+__global__ __launch_bounds__(kThreads) void permute_scan_kernel(PermuteParams p, ScanParams sp, int ep, int eq) {
     __shared__ int s_g[kMaxGroups][kMaxExperts];
+    __shared__ int s_seg[2][kThreads];
+    __shared__ float s_fseg[kThreads];
     __shared__ int s_tot[kMaxExperts];
     __shared__ int s_base[kMaxExperts];
     __shared__ int s_off[kMaxExperts + 1];
     __shared__ float s_fsum[kMaxExperts + 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int K = p.K, E = p.E, nblk = sp.nblk, b = blockIdx.x;
-    if (tid < E) {
+    // blocks per segment: at least one batch of 8 loads, so that few blocks
+    // make few segments to add up
+    const int per_e = max(8, (nblk * ep + kThreads - 1) / kThreads), nseg = (nblk + per_e - 1) / per_e;
+    const int per_q = max(8, (nblk * eq + kThreads - 1) / kThreads), nseg2 = (nblk + per_q - 1) / per_q;
+    {
+        const int e = tid & (ep - 1), seg = tid / ep, per = per_e;
+        const int b0 = seg * per, b1 = min(nblk, b0 + per), ec = min(e, E - 1);
         int tot = 0, before = 0;
-        for (int b0 = 0; b0 < nblk; b0 += 8) {
+        for (int bb = b0; bb < b1; bb += 8) {
             int v[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = sp.blkcnt[(int64_t)min(b0 + u, nblk - 1) * E + tid];
+            for (int u = 0; u < 8; ++u) v[u] = sp.blkcnt[(int64_t)min(bb + u, b1 - 1) * E + ec];
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const int c = b0 + u < nblk ? v[u] : 0;
+                const int c = bb + u < b1 ? v[u] : 0;
                 tot += c;
-                before += b0 + u < b ? c : 0;
+                before += bb + u < b ? c : 0;
             }
+        }
+        s_seg[0][tid] = tot;
+        s_seg[1][tid] = before;
+    }
+    if (b == 0) {
+        const int q = tid & (eq - 1), seg = tid / eq, per = per_q;
+        const int b0 = seg * per, b1 = min(nblk, b0 + per), qc = min(q, E);
+        float run = 0.0f;
+        for (int bb = b0; bb < b1; bb += 8) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = sp.blkstat[(int64_t)min(bb + u, b1 - 1) * (E + 1) + qc];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (bb + u < b1) run += v[u];
+        }
+        s_fseg[tid] = run;
+    }
+    __syncthreads();
+    if (tid < E) {
+        int tot = 0, before = 0;
+        for (int seg = 0; seg < nseg; ++seg) {
+            tot += s_seg[0][seg * ep + tid];
+            before += s_seg[1][seg * ep + tid];
         }
         s_tot[tid] = tot;
         s_base[tid] = before;
     } else if (b == 0 && tid >= 64 && tid - 64 <= E) {
-        const int q = tid - 64;
         float run = 0.0f;
-        for (int b0 = 0; b0 < nblk; b0 += 8) {
-            float v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = sp.blkstat[(int64_t)min(b0 + u, nblk - 1) * (E + 1) + q];
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (b0 + u < nblk) run += v[u];
-        }
-        s_fsum[q] = run;
+        for (int seg = 0; seg < nseg2; ++seg) run += s_fseg[seg * eq + tid - 64];
+        s_fsum[tid - 64] = run;
     }
     __syncthreads();
     if (tid == 0) scan_offsets_stats(sp, s_tot, s_fsum, s_off, b == 0);
@@ -1195,11 +1226,20 @@ __global__ __launch_bounds__(kThreads) void permute_scan_kernel(PermuteParams p,
     }
 }
 
+// Powers of two over the experts and over the statistics per block.
+static int pow2_at_least(int v) {
+    int q = 8;
+    while (q < v) q <<= 1;
+    return q;
+}
+bool permute_scan_fits(int nblk, int E) {
+    return nblk > 0 && nblk * pow2_at_least(E + 1) <= kThreads * 32;  // at most 32 loads per thread
+}
 hipError_t launch_permute_scan(const PermuteParams& p, const ScanParams& sp, int nblk, hipStream_t s) {
     const int RG = 64 / p.K;
-    if ((p.rows_per_block + RG - 1) / RG > kMaxGroups || nblk < 1 || nblk > kFusedScanBlocks || p.E > kMaxExperts)
+    if ((p.rows_per_block + RG - 1) / RG > kMaxGroups || p.E > kMaxExperts || !permute_scan_fits(nblk, p.E))
         return hipErrorInvalidValue;
-    permute_scan_kernel<<<nblk, kThreads, 0, s>>>(p, sp);
+    permute_scan_kernel<<<nblk, kThreads, 0, s>>>(p, sp, pow2_at_least(p.E), pow2_at_least(p.E + 1));
     return hipGetLastError();
 }
 
