@@ -211,8 +211,22 @@ bool dx_transposes(int64_t slots, int64_t E, bool padded) { return padded || slo
 // Router rows per workgroup: kRouterWaves waves x R rows x iterations, aiming
 // at a few hundred workgroups and staying within the permutation kernel's
 // group limit.
-int router_rows_per_block(int T, int E, int K) {
-    const int R = router_rows_per_wave(E);
+// Small batches: the rows of a wave share its reads of Wr, but each row's
+// LayerNorm, dot products and butterfly are issued by that wave, and 16
+// workgroups left 240 CUs idle. So a wave takes half as many rows (down to
+// one) while the grid is below kRouterShortBlocks workgroups, Wr fits LDS (it
+// is read once per workgroup) and the permutation still does the scan
+// itself. Router, event-timed us, full rows / this rule: T = 1024, d = 256,
+// E = 4 with the LayerNorm 14.3 / 7.9; T = 777, d = 1024, E = 16 with it
+// 19.5 / 13.8; T = 2048, E = 8 14.5 / 10.7; T = 3000, d = 4096, E = 8
+// 31.0 / 21.2. Up to 256 workgroups the router gains 0.4 us more on the
+// shapes next to the line and the permutation, with as many, loses 1.1
+// (T = 4095, E = 10), so the line is at 128.
+int router_rows_per_block(int T, int E, int K, int d) {
+    int R = router_rows_per_wave(E);
+    const auto blocks = [T](int r) { return (T + kRouterWaves * r - 1) / (kRouterWaves * r); };
+    if (router_wr_in_lds(E, d))
+        while (R > 1 && blocks(R) < kRouterShortBlocks && permute_scan_fits(blocks(R / 2), E)) R >>= 1;
     const int base = kRouterWaves * R;
     int iter = T / (base * 512);
     const int rg = 64 / K;
@@ -243,7 +257,9 @@ Sizes plan(const tmt_moe_desc* user, tmt_moe* m) {
     const int64_t hn = h > 0 ? h : D;
     const int64_t TK = T * K;
     const int rpb_min = kRouterWaves * router_rows_per_wave((int)E);
-    const int64_t nblk = (T + rpb_min - 1) / rpb_min;
+    // shorter router blocks (router_rows_per_block) come in less than twice kRouterShortBlocks
+    const int64_t nblk = std::max((T + rpb_min - 1) / rpb_min,
+                                  std::min<int64_t>((T + kRouterWaves - 1) / kRouterWaves, 2 * kRouterShortBlocks));
     Layout L, W;
     size_t o_logits = L.add(T * E * 4), o_probs = L.add(T * E * 4), o_lse = L.add(T * 4);
     size_t o_gate = L.add(TK * 4), o_idx = L.add(TK * 4);
@@ -471,7 +487,7 @@ int route(tmt_moe* m, hipStream_t s, int T, const uint16_t* X, const uint16_t* W
     // without the LayerNorm the logits come from the matrix cores (with the
     // canonical order for rows whose ranking that could change)
     const bool mfma = ln == nullptr && router_mfma_fits(T, E, K, d);
-    const int rpb = mfma ? kMfmaRouterRows : router_rows_per_block(T, E, K);
+    const int rpb = mfma ? kMfmaRouterRows : router_rows_per_block(T, E, K, d);
     const int nblk = T > 0 ? (T + rpb - 1) / rpb : 0;
     if (nblk > m->nblk_max) return fail(TMT_MOE_EINVAL, "internal: router block count %d > %d", nblk, m->nblk_max);
     if (nblk > 0) {

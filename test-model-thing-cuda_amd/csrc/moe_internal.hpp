@@ -26,7 +26,7 @@ struct RouterParams {
     const uint16_t* Wr;    // [E][d] bf16
     const float* bias;     // [E] or nullptr
     int T, d, E, K;
-    int rows_per_block;    // multiple of kRouterWaves * (64 / EP)
+    int rows_per_block;    // kRouterWaves x rows per wave (64 / EP, or 4, 2, 1) x iterations
     float* logits;         // [T][E]
     float* probs;          // [T][E]
     int32_t* idx;          // [T][K]
@@ -51,6 +51,7 @@ bool router_ln_fits(int E, int d);
 // Wr is staged in LDS by the router and the dX scatter when it fits in this
 // many bytes; wider routers (E*d*2 larger) are read from global memory.
 constexpr size_t kRouterWrLdsBytes = 65536;
+constexpr int kRouterShortBlocks = 128;  // router grids below this take shorter blocks
 inline bool router_wr_in_lds(int E, int d) { return (size_t)E * (size_t)d * 2 <= kRouterWrLdsBytes; }
 int router_rows_per_wave(int E);
 hipError_t launch_router(const RouterParams& p, int nblk, hipStream_t s);

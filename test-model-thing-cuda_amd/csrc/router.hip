@@ -53,11 +53,39 @@ __device__ __forceinline__ void stage_router_weights(const uint16_t* Wr, int nve
     }
 }
 
-// Route rows [row_begin, row_end) with the block's 4 waves: logits, probs,
-// top-k indices and gates, lse. Per-expert pick counts are added to s_cnt
-// (LDS atomics); each wave leaves its sum of probabilities per expert in
-// s_stat[wave][e] and its sum of lse^2 in s_stat[wave][kMaxExperts]. When
-// s_idx is given, the picks are also stored there ([row - row_begin][j]).
+// Sums of N entries per lane over the wave's 64 lanes (xor butterfly,
+// offsets 32 .. 1) as a reduce-scatter: at offset OFF while n > 1 entries are
+// left, the lanes with bit OFF set keep the upper half of their entries,
+// adding their partner's copy, so lane l ends with entry
+// sum_j bit(5 - j, l) * N / 2^(j+1) (j < log2 N); then plain butterfly steps.
+// Every addition is own + partner of the same partial trees as the full
+// butterfly, so each sum has that butterfly's bits.
+template <int OFF, int N>
+__device__ __forceinline__ void rs_sum_level(float* a, int lane) {
+    if constexpr (N > 1) {
+        const bool upper = (lane & OFF) != 0;
+#pragma unroll
+        for (int t = 0; t < N / 2; ++t) {
+            const float lo = a[t], hi = a[t + N / 2];
+            const float send = upper ? lo : hi;
+            const float keep = upper ? hi : lo;
+            a[t] = keep + xor_lane<OFF>(send);
+        }
+        rs_sum_level<OFF / 2, N / 2>(a, lane);
+    } else if constexpr (OFF >= 1) {
+        a[0] = a[0] + xor_lane<OFF>(a[0]);
+        rs_sum_level<OFF / 2, 1>(a, lane);
+    }
+}
+template <int N>
+__device__ __forceinline__ int rs_sum_entry(int lane) {
+    int idx = 0;
+#pragma unroll
+    for (int off = 32, n = N; n > 1; off >>= 1, n >>= 1)
+        if (lane & off) idx += n / 2;
+    return idx;
+}
+
 // Reduce-scatter level at offset OFF over the first 2*OFF entries of acc:
 // afterwards acc[t] (t < OFF) holds, on lane l, the sum of the entry the lane
 // keeps (t, or t + OFF when bit OFF of l is set) and its partner's copy of
@@ -86,16 +114,27 @@ __device__ __forceinline__ void reduce_scatter_level(float* acc, int lane) {
     }
 }
 
+// Route rows [row_begin, row_end) with the block's NW waves: logits, probs,
+// top-k indices and gates, lse. Per-expert pick counts are added to s_cnt
+// (LDS atomics); each wave leaves its sum of probabilities per expert in
+// s_stat[wave][e] and its sum of lse^2 in s_stat[wave][kMaxExperts].
 // NCH > 0: the rows are the block input S and pass through the LayerNorm
 // first (ln_row.hpp, the same arithmetic as ln_fwd_kernel): the wave loads
 // its R rows whole (NCH chunks of 512 elements), writes H and the row
 // statistics, and computes the logits from H as rounded to bf16, as the
 // router would read it back.
-template <int EP, int NW, int NCH = 0>
+// R rows per wave at a time: 64 / EP for full batches (64 partials per lane,
+// one per expert lane after the butterfly), fewer for small ones, whose lanes
+// end with entry rs_sum_entry(lane) and pass it on to lane row * EP + expert.
+// The first rows are on their way before `stage` (which fills wl and ends
+// with a barrier) is called, and in small batches without the LayerNorm the
+// next chunk's pieces are while a chunk's dot products run (for full batches
+// the registers cost more than the loads: with 32 expert lanes one workgroup
+// per CU instead of two, T = 10000, d = 1024, E = 32 40.7 us against 32.8).
+template <int EP, int NW, int NCH, int R, class Stage>
 __device__ __forceinline__ void route_rows(const RouterParams& p, const uint16_t* wl, int row_begin,
                                            int row_end, int* s_cnt,
-                                           float (*s_stat)[kMaxExperts + 1], int* s_idx) {
-    constexpr int R = 64 / EP;
+                                           float (*s_stat)[kMaxExperts + 1], Stage stage) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int d = p.d, E = p.E, K = p.K;
     const int e_mine = lane % EP;
@@ -104,21 +143,34 @@ __device__ __forceinline__ void route_rows(const RouterParams& p, const uint16_t
     const int nch = (d + 511) / 512;
     float psum = 0.0f, lsum = 0.0f;
 
-    for (int r0 = row_begin + wave * R; r0 < row_end; r0 += NW * R) {
+    constexpr int NP = NCH > 0 ? NCH : 1;
+    uint4 hv[R][NP];  // the rows' pieces: all NCH chunks, or (no LayerNorm) one at a time
+    auto load_chunk = [&](int r0, int c, int slot) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int row = r0 + r, k0 = c * 512 + lane * 8;
+            hv[r][slot] = make_uint4(0, 0, 0, 0);
+            if (row < row_end && k0 < d) hv[r][slot] = *reinterpret_cast<const uint4*>(p.X + (int64_t)row * d + k0);
+        }
+    };
+    constexpr bool kAhead = NCH > 0 || R * EP < 64;
+    const int first = row_begin + wave * R;
+    if constexpr (kAhead) {
+#pragma unroll
+        for (int c = 0; c < NP; ++c) load_chunk(first, c, c);
+    }
+    stage();
+
+    for (int r0 = first; r0 < row_end; r0 += NW * R) {
         float acc[R * EP];
 #pragma unroll
         for (int i = 0; i < R * EP; ++i) acc[i] = 0.0f;
+        if (kAhead && r0 != first) {
+#pragma unroll
+            for (int c = 0; c < NP; ++c) load_chunk(r0, c, c);
+        }
 
-        uint4 hv[R][NCH > 0 ? NCH : 1];  // LayerNorm: the rows' H pieces
         if constexpr (NCH > 0) {
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-#pragma unroll
-                for (int c = 0; c < NCH; ++c) {
-                    const int row = r0 + r, k0 = c * 512 + lane * 8;
-                    hv[r][c] = make_uint4(0, 0, 0, 0);
-                    if (row < row_end && k0 < d) hv[r][c] = *reinterpret_cast<const uint4*>(p.X + (int64_t)row * d + k0);
-                }
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const int row = r0 + r;
@@ -179,33 +231,37 @@ __device__ __forceinline__ void route_rows(const RouterParams& p, const uint16_t
         } else {
             for (int c = 0; c < nch; ++c) {
                 const int k0 = c * 512 + lane * 8;
-                if (k0 >= d) continue;  // this lane owns no element of the chunk
+                if (!kAhead && k0 >= d) continue;  // this lane owns no element of the chunk
+                if (!kAhead) load_chunk(r0, c, 0);
                 float xf[R][8];
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const int row = r0 + r;
-                    uint4 xv = make_uint4(0, 0, 0, 0);
-                    if (row < row_end)
-                        xv = *reinterpret_cast<const uint4*>(p.X + (int64_t)row * d + k0);
-                    unpack8(xv, xf[r]);
-                }
-                dots(k0, xf);
+                for (int r = 0; r < R; ++r) unpack8(hv[r][0], xf[r]);
+                if (kAhead && c + 1 < nch) load_chunk(r0, c + 1, 0);
+                if (k0 < d) dots(k0, xf);
             }
         }
 
         // Reduce-scatter butterfly: at offset `off` the lane keeps the half of
         // its entries whose bit log2(off) equals its own lane bit.
-        reduce_scatter_level<32>(acc, lane);
-        reduce_scatter_level<16>(acc, lane);
-        reduce_scatter_level<8>(acc, lane);
-        reduce_scatter_level<4>(acc, lane);
-        reduce_scatter_level<2>(acc, lane);
-        reduce_scatter_level<1>(acc, lane);
-        float logit = acc[0];
+        float logit;
+        if constexpr (R * EP == 64) {
+            reduce_scatter_level<32>(acc, lane);
+            reduce_scatter_level<16>(acc, lane);
+            reduce_scatter_level<8>(acc, lane);
+            reduce_scatter_level<4>(acc, lane);
+            reduce_scatter_level<2>(acc, lane);
+            reduce_scatter_level<1>(acc, lane);
+            logit = acc[0];
+        } else {
+            // entry r * EP + e is on the lanes whose upper bits are its number;
+            // lane l takes entry l % (R * EP) (lanes past R * EP hold copies)
+            rs_sum_level<32, R * EP>(acc, lane);
+            logit = __shfl(acc[0], (lane % (R * EP)) * (64 / (R * EP)), 64);
+        }
         if (p.bias != nullptr && e_valid) logit = logit + p.bias[e_mine];
 
         const int row = r0 + r_mine;
-        const bool row_valid = row < row_end;
+        const bool row_valid = r_mine < R && row < row_end;
 
         const RowPick pk = softmax_topk<EP>(logit, e_valid, e_mine, K);
         const float prob = pk.prob, lse = pk.lse;
@@ -220,7 +276,6 @@ __device__ __forceinline__ void route_rows(const RouterParams& p, const uint16_t
             if (e_mine < K) {
                 p.idx[(int64_t)row * K + e_mine] = pk.idx;
                 p.gate[(int64_t)row * K + e_mine] = pk.gate;
-                if (s_idx) s_idx[(row - row_begin) * K + e_mine] = pk.idx;
             }
             if (e_mine == 0) {
                 p.lse[row] = lse;
@@ -250,7 +305,7 @@ __device__ __forceinline__ void route_rows(const RouterParams& p, const uint16_t
 // NW waves per workgroup share one staged copy of Wr; the block statistics
 // add the waves' sums in wave order.
 // NCH > 0: the LayerNorm in front of the router is computed here (route_rows).
-template <int EP, bool WLDS, int NW, int NCH>
+template <int EP, bool WLDS, int NW, int NCH, int R = 64 / EP>
 __global__ __launch_bounds__(64 * NW) void router_kernel(RouterParams p) {
     extern __shared__ uint4 smem_w[];  // Wr [E][d] bf16 (WLDS)
     __shared__ int s_cnt[kMaxExperts];
@@ -258,14 +313,14 @@ __global__ __launch_bounds__(64 * NW) void router_kernel(RouterParams p) {
 
     const int tid = threadIdx.x;
     const int E = p.E;
-    if constexpr (WLDS) stage_router_weights(p.Wr, E * p.d / 8, smem_w);
-    if (tid < kMaxExperts) s_cnt[tid] = 0;
-    __syncthreads();
-
     const int row_begin = blockIdx.x * p.rows_per_block;
     const int row_end = min(p.T, row_begin + p.rows_per_block);
     const uint16_t* wl = WLDS ? reinterpret_cast<const uint16_t*>(smem_w) : p.Wr;
-    route_rows<EP, NW, NCH>(p, wl, row_begin, row_end, s_cnt, s_stat, nullptr);
+    route_rows<EP, NW, NCH, R>(p, wl, row_begin, row_end, s_cnt, s_stat, [&] {
+        if constexpr (WLDS) stage_router_weights(p.Wr, E * p.d / 8, smem_w);
+        if (tid < kMaxExperts) s_cnt[tid] = 0;
+        __syncthreads();
+    });
     __syncthreads();
     // Block statistics: waves added in order.
     const int b = blockIdx.x;
@@ -310,39 +365,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // then softmax_topk): bit for bit what router_kernel writes. Flagged rows
 // are taken in ascending row order, so the block statistics are
 // deterministic.
-// Sums of N entries per lane over the wave's 64 lanes (xor butterfly,
-// offsets 32 .. 1) as a reduce-scatter: at offset OFF while n > 1 entries are
-// left, the lanes with bit OFF set keep the upper half of their entries,
-// adding their partner's copy, so lane l ends with entry
-// sum_j bit(5 - j, l) * N / 2^(j+1) (j < log2 N); then plain butterfly steps.
-// Every addition is own + partner of the same partial trees as the full
-// butterfly, so each sum has that butterfly's bits.
-template <int OFF, int N>
-__device__ __forceinline__ void rs_sum_level(float* a, int lane) {
-    if constexpr (N > 1) {
-        const bool upper = (lane & OFF) != 0;
-#pragma unroll
-        for (int t = 0; t < N / 2; ++t) {
-            const float lo = a[t], hi = a[t + N / 2];
-            const float send = upper ? lo : hi;
-            const float keep = upper ? hi : lo;
-            a[t] = keep + xor_lane<OFF>(send);
-        }
-        rs_sum_level<OFF / 2, N / 2>(a, lane);
-    } else if constexpr (OFF >= 1) {
-        a[0] = a[0] + xor_lane<OFF>(a[0]);
-        rs_sum_level<OFF / 2, 1>(a, lane);
-    }
-}
-template <int N>
-__device__ __forceinline__ int rs_sum_entry(int lane) {
-    int idx = 0;
-#pragma unroll
-    for (int off = 32, n = N; n > 1; off >>= 1, n >>= 1)
-        if (lane & off) idx += n / 2;
-    return idx;
-}
-
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -878,10 +900,34 @@ hipError_t launch_router(const RouterParams& p, int nblk, hipStream_t s) {
     const int ep = router_ep(p.E);
     const int nch = p.ln_H != nullptr ? router_ln_chunks(p.E, p.d) : 0;
     if (p.ln_H != nullptr && nch == 0) return hipErrorInvalidValue;
+    const int rw = min(router_rows_per_wave(p.E), p.rows_per_block / kRouterWaves);
+    if (p.rows_per_block % (kRouterWaves * rw) != 0 || (rw != router_rows_per_wave(p.E) && (rw < 1 || !wlds)))
+        return hipErrorInvalidValue;
     dim3 grid(nblk), block(64 * kRouterWaves);
+#define TMT_ROUTER_R(EP_, NCH_, R_)                                                             \
+    if (wlds) router_kernel<EP_, true, kRouterWaves, NCH_, R_><<<grid, block, lds, s>>>(p);    \
+    else router_kernel<EP_, false, kRouterWaves, NCH_, R_><<<grid, block, 0, s>>>(p);
+// R rows per wave: fewer than 64 / EP where the batch is cut into shorter blocks
 #define TMT_ROUTER_NCH(EP_, NCH_)                                                               \
-    if (wlds) router_kernel<EP_, true, kRouterWaves, NCH_><<<grid, block, lds, s>>>(p);        \
-    else router_kernel<EP_, false, kRouterWaves, NCH_><<<grid, block, 0, s>>>(p);
+    if constexpr (EP_ < 64) {                                                                   \
+        if (rw == 1) {                                                                          \
+            router_kernel<EP_, true, kRouterWaves, NCH_, 1><<<grid, block, lds, s>>>(p);        \
+            break;                                                                              \
+        }                                                                                       \
+    }                                                                                           \
+    if constexpr (EP_ < 32) {                                                                   \
+        if (rw == 2) {                                                                          \
+            router_kernel<EP_, true, kRouterWaves, NCH_, 2><<<grid, block, lds, s>>>(p);        \
+            break;                                                                              \
+        }                                                                                       \
+    }                                                                                           \
+    if constexpr (EP_ < 16) {                                                                   \
+        if (rw == 4) {                                                                          \
+            router_kernel<EP_, true, kRouterWaves, NCH_, 4><<<grid, block, lds, s>>>(p);        \
+            break;                                                                              \
+        }                                                                                       \
+    }                                                                                           \
+    TMT_ROUTER_R(EP_, NCH_, 64 / EP_)
 #define TMT_ROUTER(EP_)                              \
     case EP_:                                        \
         if (nch == 0) { TMT_ROUTER_NCH(EP_, 0) }     \
@@ -896,6 +942,7 @@ hipError_t launch_router(const RouterParams& p, int nblk, hipStream_t s) {
         TMT_ROUTER(64)
         default: return hipErrorInvalidValue;
     }
+#undef TMT_ROUTER_R
 #undef TMT_ROUTER
 #undef TMT_ROUTER_NCH
     return hipGetLastError();

@@ -152,6 +152,22 @@ def test_layernorm_block_against_oracle(orc, T, d, E, K, h):
     check_all(g, r, E, h)
 
 
+@pytest.mark.parametrize("T,d,E,K", [
+    (2033, 512, 8, 2),   # two rows per wave, one LayerNorm chunk
+    (4066, 576, 8, 2),   # four rows per wave, two chunks
+    (1017, 1088, 9, 2),  # 16 expert lanes, one row per wave, four chunks
+    (2040, 64, 20, 3),   # 32 expert lanes, two rows per wave
+])
+def test_layernorm_block_short_router_blocks(orc, T, d, E, K):
+    """The LayerNorm in a router that takes fewer rows per wave."""
+    say(f"LayerNorm + router blocks T={T} d={d} E={E} K={K}")
+    case = make_case(T, d, E, K, 0, seed=T + E)
+    S, gamma, beta = ln_inputs(case["X"], seed=T)
+    Y0 = bf16_bits(np.zeros((T, d), np.float32))
+    check_all(run_gpu_ln(case, S, gamma, beta, K, 0, Y0, 0.01, 0.001),
+              oracle_ln(orc, case, S, gamma, beta, K, 0, Y0, 0.01, 0.001), E, 0)
+
+
 def test_layernorm_constant_rows_and_extreme_scales(orc):
     say("layernorm block: constant rows, 1e-3 and 1e3 scaled rows")
     T, d, E, K, h = 96, 256, 4, 2, 128

@@ -336,6 +336,29 @@ def test_matrix_core_router_group_walk(orc, T, d, E, K):
     near(g["z"], z, 1e-6, 1e-4, "z")
 
 
+@pytest.mark.parametrize("T,d,E,K", [
+    (65, 64, 5, 2),        # one row per wave, the last block one row long
+    (2033, 520, 8, 2),     # two rows per wave (the smallest such batch), a ragged second chunk
+    (4064, 1032, 3, 2),    # two rows per wave (the largest), a ragged third chunk
+    (4066, 128, 8, 3),     # four rows per wave
+    (8129, 64, 6, 2),      # the full eight rows
+    (2100, 136, 16, 4),    # 16 expert lanes, two rows per wave
+    (1000, 512, 32, 8),    # 32 expert lanes, one row per wave
+    (1000, 520, 31, 2),    # ... in 125 blocks
+    (2040, 64, 32, 2),     # 32 expert lanes, two rows per wave
+    (300, 3000, 12, 2),    # Wr past the LDS: full blocks at any size
+])
+def test_router_short_blocks(orc, T, d, E, K):
+    """Fewer rows per wave in small batches: the logits of every row are the
+    canonical order's bits at every block length."""
+    say(f"router blocks T={T} d={d} E={E} K={K}")
+    case = make_case(T, d, E, K, 0, seed=T + E)
+    g = run_gpu(case, K, 0, max_tokens=T + 37)
+    r = oracle_case(orc, case, K, 0)
+    check_routing(g, r, E)
+    assert np.array_equal(g["logits"].view(np.uint32), r["logits"].view(np.uint32))
+
+
 def test_runs_are_bitwise_deterministic():
     say("determinism: two identical fwd+bwd runs")
     T, d, E, K, h = 2000, 512, 8, 2, 512
