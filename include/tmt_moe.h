@@ -24,9 +24,10 @@
  * the caller's tensors directly and every device pointer must be 16-byte
  * aligned. Other widths (TMT's own tests run dim 16 and 32) run on
  * zero-padded copies at the widths rounded up to 64, kept in the handle's
- * shared workspace: each call copies its operands in and its results out
- * (a few extra small kernels), and pointers need only their natural
- * alignment (2 bytes for bf16, 4 for fp32). Zero columns add exact zeros, so
+ * shared workspace: each call copies its operands in and Y and dX out
+ * (a few extra small kernels; the weight gradients are written in place),
+ * and pointers need only their natural alignment (2 bytes for bf16, 4 for
+ * fp32). Zero columns add exact zeros, so
  * the routing is the same as at the caller's width. The MXFP4 formats keep
  * d and hidden multiples of 64.
  *
@@ -264,8 +265,8 @@ int tmt_moe_read_routing(tmt_moe* moe, void* stream, float* logits,
  *             [d] fp32 (overwritten, fixed-order sums over rows).
  * The backward needs `workspace` of at least tmt_moe_layernorm_workspace_size
  * bytes (device memory, 256-byte aligned); no call allocates. Any d >= 1
- * (rows whose width is not a multiple of 8 are read and written element by
- * element, in the same summation order); pointers 16-byte aligned. Calls
+ * (in rows whose width is not a multiple of 8 the same lanes own the same
+ * elements, so the summation order is the same); pointers 16-byte aligned. Calls
  * that share a workspace must be ordered by the caller.
  */
 int tmt_moe_layernorm_workspace_size(int32_t T, int32_t d, size_t* bytes);
