@@ -526,9 +526,9 @@ __device__ __forceinline__ void scatter_chunk(const ScatterParams& p, const int*
 // of dlogits are staged in LDS (all loads of a thread issued before its LDS
 // stores), so the per-expert loop reads only LDS.
 //
-// NI > 0 fuses the backward of the LayerNorm in front of the block
-// (d <= 512*NI): the row's gradient dH = bf16(sum) stays in registers
-// (rounded like the reference's bf16 dH), then
+// Fuses the backward of the LayerNorm in front of the block (d <= 512*NI;
+// without it scatter_rows_kernel runs): the row's gradient dH = bf16(sum)
+// stays in registers (rounded like the reference's bf16 dH), then
 //   dS = rstd * ((g - mean(g)) - xh * mean(g * xh)),  g = dH * gamma,
 //   xh = (S - mean) * rstd,
 // and every lane keeps dgamma (dH * xh) and dbeta (dH) partials of its
@@ -545,7 +545,6 @@ __global__ __launch_bounds__(kThreads) void scatter_kernel(ScatterParams p, int 
         router_dw_reduce_block(p.dw, blockIdx.x - nrow_blocks);
         return;
     }
-    constexpr int NR = NI > 0 ? NI : 1;
     constexpr bool STAGE = ROUTER && WLDS;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int d = p.d, K = p.K, E = p.E;
@@ -575,24 +574,22 @@ __global__ __launch_bounds__(kThreads) void scatter_kernel(ScatterParams p, int 
     }
     const uint16_t* wl = STAGE ? reinterpret_cast<const uint16_t*>(smem_w) : p.Wr;
 
-    float gam[NR][8], pg[NR][8], pb[NR][8];
-    if constexpr (NI > 0) {
+    float gam[NI][8], pg[NI][8], pb[NI][8];
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int c0 = i * 512 + lane * 8;
-            f32x4 g0 = f32x4{0.f, 0.f, 0.f, 0.f}, g1 = g0;
-            if (c0 < d) {
-                g0 = *reinterpret_cast<const f32x4*>(p.ln_gamma + c0);
-                g1 = *reinterpret_cast<const f32x4*>(p.ln_gamma + c0 + 4);
-            }
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                gam[i][t] = g0[t];
-                gam[i][t + 4] = g1[t];
-            }
-#pragma unroll
-            for (int t = 0; t < 8; ++t) pg[i][t] = pb[i][t] = 0.0f;
+    for (int i = 0; i < NI; ++i) {
+        const int c0 = i * 512 + lane * 8;
+        f32x4 g0 = f32x4{0.f, 0.f, 0.f, 0.f}, g1 = g0;
+        if (c0 < d) {
+            g0 = *reinterpret_cast<const f32x4*>(p.ln_gamma + c0);
+            g1 = *reinterpret_cast<const f32x4*>(p.ln_gamma + c0 + 4);
         }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            gam[i][t] = g0[t];
+            gam[i][t + 4] = g1[t];
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) pg[i][t] = pb[i][t] = 0.0f;
     }
 
     for (int r = rbeg + wave; r < rend; r += 4) {
@@ -601,92 +598,82 @@ __global__ __launch_bounds__(kThreads) void scatter_kernel(ScatterParams p, int 
         for (int j = 0; j < kMaxTopK; ++j)
             if (j < K) pos[j] = p.slot_of[(int64_t)r * K + j];
         const float* dl = s_dl + (r - rbeg) * E;
-        if constexpr (NI == 0) {
-            for (int c0 = lane * 8; c0 < d; c0 += 512) {
+        const float mean = p.ln_mean[r], rstd = p.ln_rstd[r];
+        float hv[NI][8], xs[NI][8];
+        float s1 = 0.0f, s2 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int c0 = i * 512 + lane * 8;
+            if (c0 < d) {
+                const uint4 sv = *reinterpret_cast<const uint4*>(p.ln_S + (int64_t)r * d + c0);
                 float acc[8];
                 scatter_chunk<ROUTER>(p, pos, dl, wl, c0, acc);
-                *reinterpret_cast<uint4*>(p.dX + (int64_t)r * d + c0) = pack8(acc);
-            }
-        } else {
-            const float mean = p.ln_mean[r], rstd = p.ln_rstd[r];
-            float hv[NI][8], xs[NI][8];
-            float s1 = 0.0f, s2 = 0.0f;
+                unpack8(pack8(acc), hv[i]);
+                unpack8(sv, xs[i]);
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int c0 = i * 512 + lane * 8;
-                if (c0 < d) {
-                    const uint4 sv = *reinterpret_cast<const uint4*>(p.ln_S + (int64_t)r * d + c0);
-                    float acc[8];
-                    scatter_chunk<ROUTER>(p, pos, dl, wl, c0, acc);
-                    unpack8(pack8(acc), hv[i]);
-                    unpack8(sv, xs[i]);
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        const float g = hv[i][t] * gam[i][t];
-                        const float xh = (xs[i][t] - mean) * rstd;
-                        s1 += g;
-                        s2 += g * xh;
-                        pg[i][t] += hv[i][t] * xh;
-                        pb[i][t] += hv[i][t];
-                    }
+                for (int t = 0; t < 8; ++t) {
+                    const float g = hv[i][t] * gam[i][t];
+                    const float xh = (xs[i][t] - mean) * rstd;
+                    s1 += g;
+                    s2 += g * xh;
+                    pg[i][t] += hv[i][t] * xh;
+                    pb[i][t] += hv[i][t];
                 }
             }
-            s1 = wave_sum(s1);
-            s2 = wave_sum(s2);
-            const float a = s1 / (float)d, b = s2 / (float)d;
+        }
+        s1 = wave_sum(s1);
+        s2 = wave_sum(s2);
+        const float a = s1 / (float)d, b = s2 / (float)d;
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int c0 = i * 512 + lane * 8;
-                if (c0 < d) {
-                    float out[8];
+        for (int i = 0; i < NI; ++i) {
+            const int c0 = i * 512 + lane * 8;
+            if (c0 < d) {
+                float out[8];
 #pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        const float g = hv[i][t] * gam[i][t];
-                        const float xh = (xs[i][t] - mean) * rstd;
-                        out[t] = rstd * ((g - a) - xh * b);
-                    }
-                    *reinterpret_cast<uint4*>(p.ln_dS + (int64_t)r * d + c0) = pack8(out);
+                for (int t = 0; t < 8; ++t) {
+                    const float g = hv[i][t] * gam[i][t];
+                    const float xh = (xs[i][t] - mean) * rstd;
+                    out[t] = rstd * ((g - a) - xh * b);
                 }
+                *reinterpret_cast<uint4*>(p.ln_dS + (int64_t)r * d + c0) = pack8(out);
             }
         }
     }
 
-    if constexpr (NI > 0) {
-        if (red_on_wr) __syncthreads();  // Wr reads done before it is overwritten
-        if (wave > 0) {
+    if (red_on_wr) __syncthreads();  // Wr reads done before it is overwritten
+    if (wave > 0) {
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int c0 = i * 512 + lane * 8;
-                if (c0 < d) {
-                    float* dg = s_red + (int64_t)((wave - 1) * 2) * d + c0;
-                    float* db = dg + d;
+        for (int i = 0; i < NI; ++i) {
+            const int c0 = i * 512 + lane * 8;
+            if (c0 < d) {
+                float* dg = s_red + (int64_t)((wave - 1) * 2) * d + c0;
+                float* db = dg + d;
 #pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        dg[t] = pg[i][t];
-                        db[t] = pb[i][t];
-                    }
+                for (int t = 0; t < 8; ++t) {
+                    dg[t] = pg[i][t];
+                    db[t] = pb[i][t];
                 }
             }
         }
-        __syncthreads();
-        if (wave == 0) {
-            float* outg = p.ln_partial + (int64_t)blockIdx.x * 2 * d;
-            float* outb = outg + d;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        float* outg = p.ln_partial + (int64_t)blockIdx.x * 2 * d;
+        float* outb = outg + d;
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int c0 = i * 512 + lane * 8;
-                if (c0 < d) {
-                    float g[8], b[8];
+        for (int i = 0; i < NI; ++i) {
+            const int c0 = i * 512 + lane * 8;
+            if (c0 < d) {
+                float g[8], b[8];
 #pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        g[t] = ((pg[i][t] + s_red[c0 + t]) + s_red[2 * d + c0 + t]) + s_red[4 * d + c0 + t];
-                        b[t] = ((pb[i][t] + s_red[d + c0 + t]) + s_red[3 * d + c0 + t]) + s_red[5 * d + c0 + t];
-                    }
-                    *reinterpret_cast<f32x4*>(outg + c0) = f32x4{g[0], g[1], g[2], g[3]};
-                    *reinterpret_cast<f32x4*>(outg + c0 + 4) = f32x4{g[4], g[5], g[6], g[7]};
-                    *reinterpret_cast<f32x4*>(outb + c0) = f32x4{b[0], b[1], b[2], b[3]};
-                    *reinterpret_cast<f32x4*>(outb + c0 + 4) = f32x4{b[4], b[5], b[6], b[7]};
+                for (int t = 0; t < 8; ++t) {
+                    g[t] = ((pg[i][t] + s_red[c0 + t]) + s_red[2 * d + c0 + t]) + s_red[4 * d + c0 + t];
+                    b[t] = ((pb[i][t] + s_red[d + c0 + t]) + s_red[3 * d + c0 + t]) + s_red[5 * d + c0 + t];
                 }
+                *reinterpret_cast<f32x4*>(outg + c0) = f32x4{g[0], g[1], g[2], g[3]};
+                *reinterpret_cast<f32x4*>(outg + c0 + 4) = f32x4{g[4], g[5], g[6], g[7]};
+                *reinterpret_cast<f32x4*>(outb + c0) = f32x4{b[0], b[1], b[2], b[3]};
+                *reinterpret_cast<f32x4*>(outb + c0 + 4) = f32x4{b[4], b[5], b[6], b[7]};
             }
         }
     }

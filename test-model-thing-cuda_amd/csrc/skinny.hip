@@ -17,7 +17,8 @@
 //   * the wave partials are summed in LDS in a fixed order and written with
 //     the same epilogue semantics as gemm.hip (U, SiLU(U) from the fp32 sum).
 // skinny_chunk_kernel is the main path; skinny_gemm_kernel covers reduction
-// lengths that do not split into one chunk per wave.
+// lengths that do not split into one chunk per wave; skinny_fp4_kernel
+// streams MXFP4 codes (the exact format) for small batches of any T.
 // Experts are visited in descending-count order (the scan's LPT order), so
 // the grid only spans min(E, T*K) expert ranks.
 //
