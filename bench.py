@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Benchmark of the MI355X MoE block (BASELINE.json metric).
+"""Benchmark of the MI355X MoE block.
 
 One step = forward + backward of the MoE feed-forward block on the c3
 workload: T=32768 tokens, d=1024, E=16 experts, top-4, expert hidden h=4096,
