@@ -103,6 +103,22 @@ __device__ __forceinline__ uint4 pack8(const float* f) {
     return v;
 }
 
+// A 16-byte piece that crosses the end of a row is loaded where the row ends
+// and shifted into place: the 128 bits hi:lo move down by `bits` (>= 0), zeros
+// enter from the top. 128 bits and more (a piece wholly past the end) leave
+// nothing.
+__host__ __device__ __forceinline__ void shift_piece(uint64_t& lo, uint64_t& hi, int bits) {
+    if (bits >= 128) {
+        lo = hi = 0;
+    } else if (bits >= 64) {
+        lo = hi >> (bits - 64);
+        hi = 0;
+    } else if (bits > 0) {
+        lo = (lo >> bits) | (hi << (64 - bits));
+        hi >>= bits;
+    }
+}
+
 // Non-temporal 16-byte store: an output that is written once and read by a
 // later kernel does not displace what is being reused from L2.
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));

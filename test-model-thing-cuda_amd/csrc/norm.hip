@@ -43,25 +43,21 @@ typedef unsigned u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
 // The 8 elements k0 .. k0 + 7 of a row: one 16-byte load, 16-byte aligned
 // when VEC (d, the row strides and the base pointers are multiples of 8
 // elements / 16 bytes), else at any element; elements from column d on are
-// zeros (a last piece that crosses column d is loaded where the row ends and
+// zeros (a piece that crosses column d is loaded where the row ends and
 // shifted: no load sits under a branch, so a lane's loads stay in flight
-// together). Zeros leave the row sums unchanged (x + 0 = x,
-// fma(0, 0, s) = s), so both forms give the same statistics.
-template <bool VEC>
+// together). PAST: k0 may be d or more (H's padded columns). Zeros leave the
+// row sums unchanged (x + 0 = x, fma(0, 0, s) = s), so both forms give the
+// same statistics.
+template <bool VEC, bool PAST = false>
 __device__ __forceinline__ void load_row8(const uint16_t* row, int k0, int d, float (&v)[8]) {
     if constexpr (VEC) {
         unpack8(*reinterpret_cast<const uint4*>(row + k0), v);
     } else if (d >= 8) {  // uniform
-        const int c0 = min(k0, d - 8), sh = (k0 - c0) * 16;  // bits to drop (0 .. 112; k0 < d)
+        const int c0 = min(k0, d - 8);
+        if constexpr (!PAST) __builtin_assume(k0 - c0 < 8);  // one case of the shift less
         const u32x4_any w = *reinterpret_cast<const u32x4_any*>(row + c0);
         uint64_t lo = ((uint64_t)w[1] << 32) | w[0], hi = ((uint64_t)w[3] << 32) | w[2];
-        if (sh >= 64) {
-            lo = hi >> (sh - 64);
-            hi = 0;
-        } else if (sh > 0) {
-            lo = (lo >> sh) | (hi << (64 - sh));
-            hi >>= sh;
-        }
+        shift_piece(lo, hi, (k0 - c0) * 16);
         unpack8(make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)), v);
     } else {
 #pragma unroll
@@ -136,7 +132,7 @@ __global__ __launch_bounds__(kThreads) void ln_fwd_kernel(LayerNormParams p) {
             store16<NT>(hrow + k0, hv);
         } else {
             float v[8], g[8], b[8], y[8];
-            load_row8<false>(x, k0, d, v);
+            load_row8<false, true>(x, k0, d, v);
             load_col8<false>(p.gamma, k0, d, g);
             load_col8<false>(p.beta, k0, d, b);
 #pragma unroll

@@ -1137,15 +1137,7 @@ __device__ __forceinline__ uint4 load16_edge(const V* src, int r, int c, int row
         const u32x4_any w = *reinterpret_cast<const u32x4_any*>(src + (int64_t)min(r, rows - 1) * ld + c0);
         lo = ((uint64_t)w[1] << 32) | w[0];
         hi = ((uint64_t)w[3] << 32) | w[2];
-        const int over = r < rows ? (c - c0) * (8 * (int)sizeof(V)) : 128;  // bits to drop
-        if (over >= 128) lo = hi = 0;
-        else if (over >= 64) {
-            lo = hi >> (over - 64);
-            hi = 0;
-        } else if (over > 0) {
-            lo = (lo >> over) | (hi << (64 - over));
-            hi >>= over;
-        }
+        shift_piece(lo, hi, r < rows ? (c - c0) * (8 * (int)sizeof(V)) : 128);
     } else if (r < rows) {
 #pragma unroll
         for (int t = 0; t < P; ++t) {
