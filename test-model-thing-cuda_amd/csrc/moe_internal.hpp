@@ -421,6 +421,8 @@ struct PadParams {
     void* dst[kMaxExperts];
     int64_t rows_s, cols_s, ld_s;
     int64_t rows_d, cols_d, ld_d;
+    // Set by the launcher: the destination rows of one launch.
+    int row0, nrows;
 };
 hipError_t launch_pad_copy(const PadParams& p, int nmat, int elem_bytes, hipStream_t s);
 

@@ -1165,15 +1165,16 @@ __global__ __launch_bounds__(kThreads) void pad_copy_kernel(PadParams p) {
     const V* src = static_cast<const V*>(p.src[blockIdx.y]);
     V* dst = static_cast<V*>(p.dst[blockIdx.y]);
     const uint32_t npr = (uint32_t)((p.cols_d + P - 1) / P);  // pieces per destination row
-    const uint32_t n = (uint32_t)p.rows_d * npr;               // checked by the launcher
+    const uint32_t n = (uint32_t)p.nrows * npr;                // below 2^31 (launcher)
     const uint32_t i0 = blockIdx.x * (kThreads * kPadUnroll) + threadIdx.x;
     uint32_t r[kPadUnroll], c[kPadUnroll];
     uint4 w[kPadUnroll];
 #pragma unroll
     for (int u = 0; u < kPadUnroll; ++u) {
         const uint32_t i = min(i0 + u * kThreads, n - 1);
-        r[u] = i / npr;
-        c[u] = (i - r[u] * npr) * P;
+        const uint32_t q = i / npr;
+        r[u] = (uint32_t)p.row0 + q;
+        c[u] = (i - q * npr) * P;
         w[u] = load16_edge<V>(src, (int)r[u], (int)c[u], (int)p.rows_s, (int)p.cols_s, p.ld_s);
     }
 #pragma unroll
@@ -1201,11 +1202,20 @@ hipError_t launch_pad_copy(const PadParams& p, int nmat, int elem_bytes, hipStre
     const int64_t n = p.rows_d * p.cols_d;
     if (nmat == 0 || n <= 0) return hipSuccess;
     if (p.rows_s <= 0 || p.cols_s <= 0 || (elem_bytes != 2 && elem_bytes != 4)) return hipErrorInvalidValue;
-    const int64_t per = 16 / elem_bytes, pieces = p.rows_d * ((p.cols_d + per - 1) / per);
-    const int64_t blocks = (pieces + kThreads * kPadUnroll - 1) / (kThreads * kPadUnroll);
-    if (blocks * kThreads * kPadUnroll > 0x7fffffffll) return hipErrorInvalidValue;
-    if (elem_bytes == 2) pad_copy_kernel<uint16_t><<<dim3((unsigned)blocks, nmat), kThreads, 0, s>>>(p);
-    else pad_copy_kernel<float><<<dim3((unsigned)blocks, nmat), kThreads, 0, s>>>(p);
+    // The kernel numbers the pieces of a launch in 32 bits, so matrices of more
+    // than 2^31 (experts without a hidden layer from d = 131072 on) go in
+    // several launches of whole rows.
+    const int64_t per = 16 / elem_bytes, npr = (p.cols_d + per - 1) / per, block = kThreads * kPadUnroll;
+    const int64_t rows_max = (0x7fffffffll - block) / npr;
+    if (rows_max < 1) return hipErrorInvalidValue;  // d is at most 2^20
+    for (int64_t row0 = 0; row0 < p.rows_d; row0 += rows_max) {
+        PadParams q = p;
+        q.row0 = (int)row0;
+        q.nrows = (int)std::min(rows_max, p.rows_d - row0);
+        const dim3 grid((unsigned)((q.nrows * npr + block - 1) / block), nmat);
+        if (elem_bytes == 2) pad_copy_kernel<uint16_t><<<grid, kThreads, 0, s>>>(q);
+        else pad_copy_kernel<float><<<grid, kThreads, 0, s>>>(q);
+    }
     return hipGetLastError();
 }
 

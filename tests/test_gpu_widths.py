@@ -111,6 +111,41 @@ def test_width_tiles_and_edges(orc, T, d, E, K, h):
     test_width_matches_explicit_padding(T, d, E, K, h)
 
 
+def test_width_weights_beyond_one_padding_launch():
+    """A weight matrix of more than 2^31 16-byte pieces (34 GB: a reference
+    expert at d = 131100) is padded in several launches, the second of which
+    holds the last 128 of 131136 rows. Every column of Y against fp32
+    products: the bf16 roundings of U and Y (2^-9 relative each) stay under
+    5e-3 relative L2, over the last 512 columns alone too."""
+    T, d = 65, 131100
+    say(f"width T={T} d={d} E=1 h=0 (one weight matrix of {2 * d * d / 1e9:.1f} GB)")
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 140e9:
+        pytest.skip("needs 140 GB of free device memory")
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    X = torch.randn(T, d, generator=gen, device="cuda").to(torch.bfloat16)
+    W = torch.empty(1, d, d, dtype=torch.bfloat16, device="cuda")
+    rows = 4096
+    for i in range(0, d, rows):
+        W[0, i:i + rows].normal_(0.0, d ** -0.5, generator=gen)
+    Y = torch.zeros(T, d, dtype=torch.bfloat16, device="cuda")
+    m = tmt_moe.MoE(T, d, 1, 1, 0)
+    try:
+        m.forward(X, None, W, None, Y, beta=0.0)
+        torch.cuda.synchronize()
+    finally:
+        m.close()
+    want = torch.cat([torch.nn.functional.silu(X.float() @ W[0, i:i + rows].float().t())
+                      for i in range(0, d, rows)], dim=1).cpu().numpy()
+    del W
+    torch.cuda.empty_cache()
+    got = host_f32(Y)
+    for name, cols in (("all columns", slice(0, d)), ("the last 512", slice(d - 512, d))):
+        err = rel_l2(got[:, cols], want[:, cols])
+        say(f"  Y rel-L2 over {name} {err:.2e}")
+        assert err <= 5e-3
+
+
 @pytest.mark.parametrize("T,d,E,K,h", [
     (14, 16, 2, 2, 0),
     (14, 16, 1, 1, 0),
