@@ -17,6 +17,7 @@ import pytest
 import torch
 
 import tmt_moe
+from launched_kernels import launched_kernels
 from synthetic import CONFIGS, bf16_bits, bf16_to_f32, make_case, mxfp4_experts
 from torch_ref import moe_reference
 
@@ -96,7 +97,7 @@ def test_mxfp4_against_oracle(orc, fmt, T, d, E, K, h):
     (1, 1024, 32, 4, 4096),    # one token: tables from the router, one row per expert, 16 waves in DOWN
     (64, 1024, 32, 4, 256),    # the largest decode batch
     (8, 320, 64, 8, 64),       # 64 experts; K = 320 (a partial chunk) and K = 64 (a quarter of one)
-    (33, 256, 2, 2, 4352),     # 33 rows per expert (three row blocks); DOWN over 17 chunks on 16 waves
+    (33, 256, 2, 2, 4352),     # 33 rows per expert (three row blocks); DOWN over 17 chunks on 8 waves
     (40, 192, 1, 1, 1088),     # one expert: slot = token, five waves in DOWN
     (2, 2048, 4, 1, 2304),     # 8 waves in UP, 9 in DOWN
 ])
@@ -116,6 +117,55 @@ def test_mxfp4_decode_against_oracle(orc, T, d, E, K, h):
     err = rel_l2(g["Y"], r["Y"])
     say(f"  Y rel-L2 {err:.2e}")
     assert err <= 6e-3
+
+
+def gemm_variants(T, d, E, K, h):
+    """The expert GEMM kernels an exact-format forward of this shape launches."""
+    z8 = lambda *s: torch.zeros(s, dtype=torch.uint8, device="cuda")
+    z16 = lambda *s: torch.zeros(s, dtype=torch.bfloat16, device="cuda")
+    X, Wr, Y = z16(T, d), z16(E, d), z16(T, d)
+    wu, su, wd, sd = z8(E, h, d // 2), z8(E, d // 32, h), z8(E, d, h // 2), z8(E, h // 32, d)
+    m = tmt_moe.MoE(T, d, E, K, h, weight_format=tmt_moe.WEIGHTS_MXFP4)
+    try:
+        call = lambda: m.forward_mxfp4(X, Wr, wu, su, wd, sd, Y)
+        call()
+        names = launched_kernels(call)
+    finally:
+        m.close()
+    return [n for n in names if "skinny" in n or "gemm" in n]
+
+
+# Name of each variant: GEMM_UP_FP4 is kind 6, GEMM_DOWN_FP4 kind 7.
+def tiles(kind):
+    return f"grouped_gemm_kernelILi{kind}E"
+
+
+def streamed(kind, waves, row_blocks, one_chunk):
+    return f"skinny_fp4_kernelILi{kind}ELi{waves}ELi{row_blocks}ELb{int(one_chunk)}EE"
+
+
+@pytest.mark.parametrize("T,d,E,K,h,up,down", [
+    # batches whose tables come from the permutation (more than 64 tokens)
+    (100, 1024, 32, 4, 256, streamed(6, 4, 1, True), streamed(7, 4, 1, True)),     # 16 rows per workgroup
+    (70, 256, 32, 4, 2560, streamed(6, 4, 1, True), streamed(7, 16, 1, True)),     # ... and 10 waves in DOWN
+    (200, 1280, 32, 4, 128, streamed(6, 8, 2, True), streamed(7, 4, 2, True)),     # 32 rows, 5 waves in UP
+    (300, 256, 32, 4, 4096, streamed(6, 4, 2, True), streamed(7, 8, 2, False)),    # 32 rows, 16 chunks on 8 waves
+    # decode batches, tables from the pick table
+    (24, 256, 8, 2, 512, streamed(6, 4, 2, True), streamed(7, 4, 2, True)),        # 17 to 32 tokens
+    (8, 256, 4, 2, 4352, streamed(6, 4, 1, True), streamed(7, 8, 1, False)),       # 17 chunks on 8 waves
+    # 256 x 256 tiles
+    (8192, 1024, 8, 2, 1984, tiles(6), tiles(7)),  # UP: 192 columns in the last column tile, two rounds and a rest
+    (7503, 448, 4, 4, 320, tiles(6), tiles(7)),    # last column tiles of 64 and 192 columns, 7 and 5 K steps
+    (14000, 320, 4, 4, 192, tiles(6), streamed(7, 4, 2, True)),  # 192 columns in all; DOWN streams
+])
+def test_mxfp4_gemm_variants_against_oracle(orc, T, d, E, K, h, up, down):
+    """The exact format on each variant of its two GEMMs, by name (so that a
+    change of the rule that chooses them cannot leave one untested), with the
+    bound of the decode batches above."""
+    say(f"mxfp4 variants T={T} d={d} E={E} K={K} h={h}")
+    got = gemm_variants(T, d, E, K, h)
+    assert len(got) == 2 and up in got[0] and down in got[1], got
+    test_mxfp4_decode_against_oracle(orc, T, d, E, K, h)
 
 
 def test_mxfp4_mx_tracks_exact_format(orc):
