@@ -50,21 +50,19 @@
 namespace tmt {
 namespace {
 
-constexpr int BM = kGemmTileRows;  // tile rows of the large-problem kernels (TBM: the tile's own)
+constexpr int kLarge = kGemmTileRows;  // tile of the large-problem kernels
 
-// Tile geometry. BK_ is the K depth of one LDS stage (32 or 64), NST the
-// number of stages in the ring, BM_ x BN_ the tile and NWM_ the waves along
-// M (2 x NWM_ waves per workgroup).
-template <int BK_, int NST, int BN_, int NWM_ = 2, int BM_ = 256>
+// Tile geometry: TILE x TILE outputs (256 or 128) on 4 waves in 2 x 2. BK_ is
+// the K depth of one LDS stage (32 or 64), NST the number of stages in the
+// ring.
+template <int BK_, int NST, int TILE>
 struct Geo {
-    static constexpr int BM = BM_;
+    static constexpr int BM = TILE, BN = TILE;
     static constexpr int BK = BK_;
-    static constexpr int NSTAGE = NST;
-    static constexpr int BN = BN_;
-    static constexpr int NWM = NWM_, NW = 2 * NWM_, NT = 64 * NW;  // waves, threads
-    static constexpr int WTM = BM / NWM, MI = WTM / 32;  // wave tile rows
+    static constexpr int NW = 4, NT = 64 * NW;         // waves, threads
+    static constexpr int WTM = BM / 2, MI = WTM / 32;  // wave tile rows
     static constexpr int WTN = BN / 2, NJ = WTN / 32;  // wave tile columns
-    static constexpr int EPR = NWM == 2 ? 64 : 32;     // epilogue rows per wave and pass
+    static constexpr int EPR = 64;                     // epilogue rows per wave and pass
     static constexpr int KCH = BK / 8;                 // 16-byte chunks per K-contiguous row
     static constexpr int OPND_A = BM * BK;             // bf16 elements of the A tile
     static constexpr int OPND_B = BN * BK;             // bf16 elements of the B tile
@@ -74,7 +72,7 @@ struct Geo {
     static constexpr int DMA_PER_TILE = DMA_A + DMA_B;
     static constexpr int KC_ROWS = 1024 / (2 * BK);    // K-contiguous rows per wave load
     static constexpr int STEPS = BK / 16;              // MFMA k16 steps per stage
-    static constexpr int WGS = (BN == 256 && BM == 256) || (BK == 64 && NST > 2) ? 1 : 2;  // workgroups per CU
+    static constexpr int WGS = TILE == 256 || (BK == 64 && NST > 2) ? 1 : 2;  // workgroups per CU
     // the epilogue's fp32 staging ([EPR][WTN] per wave); the kernel sizes the
     // ring (single or split) and checks the total
     static constexpr int EPI = NW * EPR * WTN * 4;
@@ -188,7 +186,7 @@ __device__ __forceinline__ void list_tile(int j, int mtiles, int ntn, int rows, 
 // M tiles per block of the activation GEMMs' list.
 __device__ __forceinline__ int list_rows(int ntn) { return ntn >= 8 ? 4 : 32 / ntn; }
 
-// Split-K of the last round (GEMM_DOWN / GEMM_DX, tiles 256 x BN, one
+// Split-K of the last round (GEMM_DOWN / GEMM_DX, tiles 256 x 256, one
 // workgroup per CU). Of the launch's tiles, F (a multiple of the W resident
 // workgroups) fill whole rounds. The R tiles left would run as one short
 // round on R CUs while the rest idle, so each is cut into S parts along K
@@ -199,10 +197,9 @@ __device__ __forceinline__ int list_rows(int ntn) { return ntn >= 8 ? 4 : 32 / n
 struct SplitPlan {
     int F = 0, R = 0, S = 1, chunk = 0;  // chunk: reduction length of a part
 };
-template <int TBM = BM>
 __device__ __forceinline__ int act_mtiles(const GemmParams& p) {
     int mt = 0;
-    for (int ee = 0; ee < p.E; ++ee) mt += (p.offsets[ee + 1] - p.offsets[ee] + TBM - 1) / TBM;
+    for (int ee = 0; ee < p.E; ++ee) mt += (p.offsets[ee + 1] - p.offsets[ee] + kLarge - 1) / kLarge;
     return mt;
 }
 template <int BK>
@@ -220,56 +217,54 @@ __device__ __forceinline__ SplitPlan split_plan(const GemmParams& p, int tiles) 
     sp.chunk = ((nk + S - 1) / S) * BK;
     return sp;
 }
-// Expert segment of activation M tile mt (TBM rows per tile): expert, first
+// Expert segment of activation M tile mt (256 rows per tile): expert, first
 // slot, rows (e < 0: none).
-template <int TBM = BM>
 __device__ __forceinline__ void act_tile(const GemmParams& p, int mt, int& e, int& row0, int& rows) {
     e = -1;
     int t0 = 0;
     for (int ee = 0; ee < p.E; ++ee) {
         const int beg = p.offsets[ee], end = p.offsets[ee + 1];
-        const int tiles = (end - beg + TBM - 1) / TBM;
+        const int tiles = (end - beg + kLarge - 1) / kLarge;
         if (mt < t0 + tiles) {
             e = ee;
-            row0 = beg + (mt - t0) * TBM;
-            rows = min(TBM, end - row0);
+            row0 = beg + (mt - t0) * kLarge;
+            rows = min(kLarge, end - row0);
             return;
         }
         t0 += tiles;
     }
 }
 
-// Split rings (A in NST slots, B in NST - 1) for K = 64 tiles of the
-// activation GEMMs on 256 x 256 tiles.
-template <int KIND, int BK, int BN, int NWM, int TBM = BM>
-constexpr bool split_ring() {
-    return BK == 64 && BN == 256 && NWM == 2 && TBM == 256 && !Traits<KIND>::group_k;
-}
-
-// Persistent kernels: the split-ring GEMMs (every tile of a launch has the
-// same K, so a static schedule stays balanced) run one workgroup per CU that
+// Split rings (A in 3 slots, B in 2) of K = 64: the activation GEMMs on
+// 256 x 256 tiles. Those kernels are persistent (every tile of a launch has
+// the same K, so a static schedule stays balanced): one workgroup per CU
 // walks the tiles vb = blockIdx.x, blockIdx.x + gridDim.x, ... . A tile's
 // first operand loads then go out while the previous tile's epilogue stores
 // drain, and the per-workgroup launch and set-up cost is paid once per CU
 // instead of once per tile. vb keeps the launch-order meaning of blockIdx.x
 // (gridDim.x is a multiple of 8 whenever it is below the tile count, so vb
 // runs on XCD vb % 8 as the tile map assumes).
-template <int KIND, int BK, int BN, int NWM, int TBM = BM>
-constexpr bool persistent_tiles() {
-    return split_ring<KIND, BK, BN, NWM, TBM>();
+template <int KIND, int TILE>
+constexpr bool split_ring() {
+    return TILE == 256 && !Traits<KIND>::group_k;
 }
 
+// MXFP4 B operand (split rings of K = 64 only): per stage 256 rows x 32 bytes
+// of codes, then one 1 KiB copy per wave of the tile's row scales (lanes 0-15
+// load the first 32-block's, lanes 16-31 the second's).
+constexpr int kFp4Codes = 256 * 32, kFp4Scales = 4 * 1024;
+// bf16 elements of a B tile's slot.
+template <int KIND, int BK, int NST, int TILE>
+constexpr int b_slot_elems() {
+    return Traits<KIND>::b_fp4 ? (kFp4Codes + kFp4Scales) / 2 : Geo<BK, NST, TILE>::OPND_B;
+}
 // LDS of one workgroup: the operand ring, or the epilogue's fp32 staging if
-// larger (MXFP4 B operand per stage: 256 rows x BK/2 bytes of codes, then
-// one 1 KiB copy per wave of the row scales).
-template <int KIND, int BK_, int NST, int BN_, int NWM_, int BM_>
+// larger.
+template <int KIND, int BK, int NST, int TILE>
 constexpr int gemm_lds_bytes() {
-    using Gm = Geo<BK_, NST, BN_, NWM_, BM_>;
-    constexpr int codes = 256 * (BK_ / 2), scales = 4 * 1024;
-    constexpr int stage = Traits<KIND>::b_fp4 ? Gm::OPND_A + (codes + scales) / 2 : Gm::STAGE;
-    constexpr int bslot = Traits<KIND>::b_fp4 ? (codes + scales) / 2 : Gm::OPND_B;
-    constexpr int ring = split_ring<KIND, BK_, BN_, NWM_, BM_>() ? (NST * Gm::OPND_A + (NST - 1) * bslot) * 2
-                                                                : NST * stage * 2;
+    using Gm = Geo<BK, NST, TILE>;
+    constexpr int ring = split_ring<KIND, TILE>() ? (NST * Gm::OPND_A + (NST - 1) * b_slot_elems<KIND, BK, NST, TILE>()) * 2
+                                                  : NST * Gm::STAGE * 2;
     return ring > Gm::EPI ? ring : Gm::EPI;
 }
 
@@ -278,34 +273,24 @@ constexpr int gemm_lds_bytes() {
 // experts' activation tiles (unused by the weight-gradient kinds). lds_raw:
 // the workgroup's gemm_lds_bytes() of LDS, declared by the kernel (measured:
 // DOWN and DX about 1% faster at c3 than with the array declared here).
-template <int KIND, bool DUAL, int BK_, int NST, int BN_, int NWM_ = 2, int BM_ = 256>
+template <int KIND, bool DUAL, int BK_, int NST, int TILE>
 __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int vb, const ExpertTiles& et,
                                                   uint4* lds_raw) {
     using Tr = Traits<KIND>;
-    using Gm = Geo<BK_, NST, BN_, NWM_, BM_>;
+    using Gm = Geo<BK_, NST, TILE>;
     constexpr int BM = Gm::BM;
-    constexpr int BK = Gm::BK, NSTAGE = Gm::NSTAGE, BN = Gm::BN, WTN = Gm::WTN, NJ = Gm::NJ;
+    constexpr int BK = Gm::BK, BN = Gm::BN, WTN = Gm::WTN, NJ = Gm::NJ;
     constexpr int WTM = Gm::WTM, MI = Gm::MI, NT = Gm::NT, EPR = Gm::EPR;
-    constexpr int OPND_A = Gm::OPND_A, OPND_B = Gm::OPND_B;
-    constexpr int DMA_A = Gm::DMA_A, DMA_B = Gm::DMA_B;
-    constexpr bool kSplit = split_ring<KIND, BK_, BN_, NWM_, BM_>();
-    static_assert(!kSplit || NST == 3, "split rings: 3 A slots and 2 B slots");
-    static_assert(BM == 256 || (BN == 128 && NWM_ == 2 && !Tr::b_fp4), "128-row tiles: 128 columns, 4 waves, bf16");
-    // MXFP4 B operand per tile: 256 rows x BK/2 bytes of codes, then one 1 KiB
-    // copy per wave of the tile's row scales (one 32-block at BK = 32, two at
-    // BK = 64: lanes 16-31 load the second block's).
-    static_assert(!Tr::b_fp4 || (BN == 256 && NWM_ == 2 && (BK == 32 || kSplit)), "MXFP4 tiles: 256 columns, 4 waves");
-    constexpr int FP4_CODES = 256 * (BK / 2), FP4_SCALES = 4 * 1024;
-    constexpr int STAGE = Tr::b_fp4 ? OPND_A + (FP4_CODES + FP4_SCALES) / 2 : Gm::STAGE;  // bf16 elements
-    constexpr int DMA_PER_TILE = Tr::b_fp4 ? DMA_A + 2 : Gm::DMA_PER_TILE;
+    constexpr int OPND_A = Gm::OPND_A, STAGE = Gm::STAGE;
+    constexpr int DMA_A = Gm::DMA_A, DMA_B = Gm::DMA_B, DMA_PER_TILE = Gm::DMA_PER_TILE;
+    constexpr bool kSplit = split_ring<KIND, TILE>();
+    static_assert(!kSplit || (NST == 3 && BK == 64), "split rings: 3 A slots and 2 B slots of K = 64");
+    static_assert(!Tr::b_fp4 || kSplit, "MXFP4 tiles: split rings");
     // split rings: B slot size (bf16 elements) and wave loads per B tile
-    constexpr int B_SLOT = Tr::b_fp4 ? (FP4_CODES + FP4_SCALES) / 2 : OPND_B;
-    constexpr int DMA_BT = Tr::b_fp4 ? FP4_CODES / 1024 / 4 + 1 : DMA_B;
+    constexpr int B_SLOT = b_slot_elems<KIND, BK_, NST, TILE>();
+    constexpr int DMA_BT = Tr::b_fp4 ? kFp4Codes / 1024 / 4 + 1 : DMA_B;
     constexpr int KCH = Gm::KCH, KC_ROWS = Gm::KC_ROWS, STEPS = Gm::STEPS;
-    constexpr int RING = kSplit ? (NST * OPND_A + (NST - 1) * B_SLOT) * 2 : NSTAGE * STAGE * 2;
-    constexpr int LDS_TOTAL = RING > Gm::EPI ? RING : Gm::EPI;
-    static_assert(LDS_TOTAL * Gm::WGS <= 160 * 1024, "LDS ring too large");
-    static_assert(LDS_TOTAL == gemm_lds_bytes<KIND, BK_, NST, BN_, NWM_, BM_>(), "LDS size of the kernel's array");
+    static_assert(gemm_lds_bytes<KIND, BK_, NST, TILE>() * Gm::WGS <= 160 * 1024, "LDS ring too large");
     uint16_t* lds = reinterpret_cast<uint16_t*>(lds_raw);
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -451,36 +436,28 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
             b_k[i] = k;
         }
     }
-    // MXFP4: wave w loads the codes of rows 64w + lane (16 bytes per tile) and
-    // its own copy of the tile's 256 row scales (lane l -> rows 16(l%16)..+15;
-    // row groups past N are clamped to the tile's first group).
-    // With split rings (BK = 64) lane pair (2m, 2m+1) loads the 32 code bytes
-    // of row m (two 16-byte halves, swapped in LDS when bit 3 of m is set) and
-    // lanes 16-31 load the second scale block.
-    const uint8_t* q_ptr = nullptr;
-    const uint8_t* q2_ptr[2] = {nullptr, nullptr};
+    // MXFP4: lane pair (2m, 2m+1) loads the 32 code bytes of row m (two 16-byte
+    // halves, swapped in LDS when bit 3 of m is set); every wave loads its own
+    // copy of the tile's 256 row scales of both 32-blocks (lane l: rows
+    // 16(l%16)..+15 of block l/16; row groups past N are clamped to the tile's
+    // first group).
+    const uint8_t* q_ptr[2] = {nullptr, nullptr};
     const uint8_t* sc_ptr = nullptr;
     if constexpr (Tr::b_fp4) {
         const int g = nt * BN + 16 * (lane & 15);
-        if constexpr (kSplit) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int sl = (wave * 2 + i) * 64 + lane, m = sl >> 1;
-                const int half = (sl & 1) ^ ((m >> 3) & 1);
-                q2_ptr[i] = p.wq[e] + (int64_t)min(nt * BN + m, p.N - 1) * (p.K / 2) + half * 16;
-            }
-            sc_ptr = p.wsc[e] + (int64_t)((lane >> 4) & 1) * p.N + (g < p.N ? g : nt * BN);
-        } else {
-            const int n = min(nt * BN + 64 * wave + lane, p.N - 1);
-            q_ptr = p.wq[e] + (int64_t)n * (p.K / 2);
-            sc_ptr = p.wsc[e] + (g < p.N ? g : nt * BN);
+        for (int i = 0; i < 2; ++i) {
+            const int sl = (wave * 2 + i) * 64 + lane, m = sl >> 1;
+            const int half = (sl & 1) ^ ((m >> 3) & 1);
+            q_ptr[i] = p.wq[e] + (int64_t)min(nt * BN + m, p.N - 1) * (p.K / 2) + half * 16;
         }
+        sc_ptr = p.wsc[e] + (int64_t)((lane >> 4) & 1) * p.N + (g < p.N ? g : nt * BN);
     }
     const uint32_t lds0 = lds_addr(lds);
     // bf16 element offsets of tile t's A and B operand tiles in LDS
-    auto a_slot = [&](int t) -> int { return kSplit ? (t % NST) * OPND_A : (t % NSTAGE) * STAGE; };
+    auto a_slot = [&](int t) -> int { return kSplit ? (t % NST) * OPND_A : (t % NST) * STAGE; };
     auto b_slot = [&](int t) -> int {
-        return kSplit ? NST * OPND_A + (t % (NST - 1)) * B_SLOT : (t % NSTAGE) * STAGE + OPND_A;
+        return kSplit ? NST * OPND_A + (t % (NST - 1)) * B_SLOT : (t % NST) * STAGE + OPND_A;
     };
     // Wave load i of tile t's A / B operand (t clamped to the last real tile
     // so the per-tile load count stays constant).
@@ -493,18 +470,18 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
         const int k0 = kbeg + min(t, nk - 1) * BK;
         if constexpr (Tr::b_fp4) {
             const uint32_t sb = lds0 + (uint32_t)b_slot(t) * 2u;
-            if (i < DMA_BT - 1) dma16(q2_ptr[i] + k0 / 2, sb + (uint32_t)(wave * (DMA_BT - 1) + i) * 1024u);
-            else dma16(sc_ptr + (int64_t)(k0 / 32) * p.N, sb + FP4_CODES + (uint32_t)wave * 1024u);
+            if (i < DMA_BT - 1) dma16(q_ptr[i] + k0 / 2, sb + (uint32_t)(wave * (DMA_BT - 1) + i) * 1024u);
+            else dma16(sc_ptr + (int64_t)(k0 / 32) * p.N, sb + kFp4Codes + (uint32_t)wave * 1024u);
         } else {
             const uint16_t* gb = Tr::b_kc ? b_ptr[i] + k0 : b_ptr[i] + (int64_t)min(k0 + b_k[i], kend - 1) * p.ldb;
             dma16(gb, lds0 + (uint32_t)b_slot(t) * 2u + (uint32_t)(wave * DMA_B + i) * 1024u);
         }
     };
-    // Issue the 8 wave loads of K tile t (clamped to the last real tile so the
-    // per-tile load count stays constant) into stage t % NSTAGE.
+    // One ring: issue the wave loads of K tile t (clamped to the last real tile
+    // so the per-tile load count stays constant) into stage t % NST.
     auto dma_tile = [&](int t) {
         const int k0 = kbeg + min(t, nk - 1) * BK;  // first reduction index of the tile
-        const uint32_t sbase = lds0 + (uint32_t)((t % NSTAGE) * STAGE) * 2u;
+        const uint32_t sbase = lds0 + (uint32_t)((t % NST) * STAGE) * 2u;
 #pragma unroll
         for (int i = 0; i < DMA_A; ++i) {
             const uint32_t qoff = (uint32_t)(wave * DMA_A + i) * 1024u;
@@ -512,24 +489,18 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
                                           : a_ptr[i] + (int64_t)min(k0 + a_k[i], kend - 1) * p.lda;
             dma16(ga, sbase + qoff);
         }
-        if constexpr (!Tr::b_fp4) {
 #pragma unroll
-            for (int i = 0; i < DMA_B; ++i) {
-                const uint32_t qoff = (uint32_t)(wave * DMA_B + i) * 1024u;
-                const uint16_t* gb = Tr::b_kc ? b_ptr[i] + k0
-                                              : b_ptr[i] + (int64_t)min(k0 + b_k[i], kend - 1) * p.ldb;
-                dma16(gb, sbase + OPND_A * 2u + qoff);
-            }
-        } else {
-            const int kb = k0 / 32;  // scale block of this tile
-            dma16(q_ptr + kb * 16, sbase + OPND_A * 2u + (uint32_t)wave * 1024u);
-            dma16(sc_ptr + (int64_t)kb * p.N, sbase + OPND_A * 2u + FP4_CODES + (uint32_t)wave * 1024u);
+        for (int i = 0; i < DMA_B; ++i) {
+            const uint32_t qoff = (uint32_t)(wave * DMA_B + i) * 1024u;
+            const uint16_t* gb = Tr::b_kc ? b_ptr[i] + k0
+                                          : b_ptr[i] + (int64_t)min(k0 + b_k[i], kend - 1) * p.ldb;
+            dma16(gb, sbase + OPND_A * 2u + qoff);
         }
     };
     // Load `idx` of dma_tile(t) on its own, for interleaving with the MFMAs.
     auto dma_one = [&](int t, int idx) {
         const int k0 = kbeg + min(t, nk - 1) * BK;
-        const uint32_t sbase = lds0 + (uint32_t)((t % NSTAGE) * STAGE) * 2u;
+        const uint32_t sbase = lds0 + (uint32_t)((t % NST) * STAGE) * 2u;
         if (idx < DMA_A) {
             const uint32_t qoff = (uint32_t)(wave * DMA_A + idx) * 1024u;
             const uint16_t* ga = Tr::a_kc ? a_ptr[idx] + k0
@@ -549,7 +520,7 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
         if constexpr (Tr::group_k) {
             const int kvalid = kend - (kbeg + t * BK);
             if (kvalid < BK) {
-                uint16_t* st = lds + (t % NSTAGE) * STAGE;
+                uint16_t* st = lds + (t % NST) * STAGE;
                 const int na = (BK - kvalid) * (BM / 8), nb = (BK - kvalid) * (BN / 8);  // 16-byte vectors
                 for (int v = tid; v < na + nb; v += NT) {
                     if (v < na) *reinterpret_cast<uint4*>(st + kvalid * BM + v * 8) = make_uint4(0, 0, 0, 0);
@@ -587,23 +558,17 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
         }
         return make_uint4(w[0], w[1], w[2], w[3]);
     };
-    // MXFP4: lane reads 4 bytes (8 codes: k = 16s + 8(lane/32) .. +7) of row
-    // rbase + lane%32 and that row's scale from its wave's copy, and expands
-    // them to a bf16 fragment.
+    // MXFP4: lane reads 4 bytes (8 codes: k = 16s + 8(lane/32) .. +7, byte
+    // 8s + 4(lane/32) of the row's 32) of row rbase + lane%32 and that row's
+    // scale from its wave's copy, and expands them to a bf16 fragment.
     auto read_fp4 = [&](const uint16_t* tB, int rbase, int s) {
         const uint8_t* codes = reinterpret_cast<const uint8_t*>(tB);
-        const uint8_t* scales = codes + FP4_CODES + wave * 1024;
+        const uint8_t* scales = codes + kFp4Codes + wave * 1024;
         const int r = rbase + (lane & 31);
-        if constexpr (kSplit) {
-            // k = 16s + 8(lane/32) .. +7: byte 8s + 4(lane/32) of the row's 32
-            const int blk = s >> 1, within = (8 * s + 4 * (lane >> 5)) & 15;
-            const uint32_t w = *reinterpret_cast<const uint32_t*>(
-                codes + r * 32 + ((blk ^ ((lane >> 3) & 1)) * 16) + within);
-            return dequant8(w, scales[blk * 256 + r]);
-        } else {
-            const uint32_t w = *reinterpret_cast<const uint32_t*>(codes + r * 16 + (2 * s + (lane >> 5)) * 4);
-            return dequant8(w, scales[r]);
-        }
+        const int blk = s >> 1, within = (8 * s + 4 * (lane >> 5)) & 15;
+        const uint32_t w = *reinterpret_cast<const uint32_t*>(
+            codes + r * 32 + ((blk ^ ((lane >> 3) & 1)) * 16) + within);
+        return dequant8(w, scales[blk * 256 + r]);
     };
     auto load_frag = [&](Frag& f, int t, int s) {
         const uint16_t* tA = lds + a_slot(t);
@@ -630,7 +595,7 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
     // they issue. Measured on the c3 shapes: DOWN 1.115 -> 1.070 ms, UP and
     // DACT about 0.5% faster; DX (+6.6%) and the weight-gradient GEMMs
     // (+1-2.5%) keep the loads in one batch.
-    constexpr bool kSpreadDma = !Tr::b_fp4 && (KIND == GEMM_DOWN || KIND == GEMM_UP || KIND == GEMM_DACT);
+    constexpr bool kSpreadDma = KIND == GEMM_DOWN || KIND == GEMM_UP || KIND == GEMM_DACT;
     auto mma_dma = [&](const Frag& f, int t) {
         constexpr int NM = MI * NJ;
         int dq = 0;
@@ -664,11 +629,11 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
     // ---- main loop ----------------------------------------------------------
     // Iteration kt runs the STEPS k16 steps of tile kt. Every step first reads
     // the next step's fragments; the first step also issues the loads of
-    // tile kt + NSTAGE - 1. Before the last step the wave waits for its loads
+    // tile kt + NST - 1. Before the last step the wave waits for its loads
     // of tile kt+1 and the workgroup synchronises (all loads of tile kt+1 are
     // visible, and every wave is done reading the stage that the next
     // iteration refills); the last step then prefetches step 0 of tile kt+1.
-    constexpr int VM_AHEAD = (NSTAGE - 2) * DMA_PER_TILE;
+    constexpr int VM_AHEAD = (NST - 2) * DMA_PER_TILE;
     if constexpr (kSplit) {
         // Split rings. Iteration kt multiplies tile kt in STEPS k16 steps;
         // the loads of B(kt+1) and then A(kt+2) are spread over the MFMAs of
@@ -732,8 +697,8 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
         }
     } else if (nk > 0) {
 #pragma unroll
-        for (int t = 0; t < NSTAGE - 1; ++t) dma_tile(t);
-        wait_vm<(NSTAGE >= 2 ? VM_AHEAD : 0)>();
+        for (int t = 0; t < NST - 1; ++t) dma_tile(t);
+        wait_vm<VM_AHEAD>();
         __syncthreads();
         if (nk == 1) {
             zero_tail(0);
@@ -747,11 +712,11 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
                 load_frag(f[(s + 1) & 1], kt, s + 1);
                 if constexpr (kSpreadDma) {
                     if (s == 0) {
-                        mma_dma(f[0], kt + NSTAGE - 1);
+                        mma_dma(f[0], kt + NST - 1);
                         continue;
                     }
                 } else {
-                    if (s == 0) dma_tile(kt + NSTAGE - 1);
+                    if (s == 0) dma_tile(kt + NST - 1);
                 }
                 mma(f[s & 1]);
 #pragma unroll
@@ -762,11 +727,7 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
                 __builtin_amdgcn_sched_group_barrier(0x008, MI * NJ / 2, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if constexpr (NSTAGE == 2) {
-                wait_vm<0>();
-            } else {
-                wait_vm<VM_AHEAD>();
-            }
+            wait_vm<VM_AHEAD>();
             __syncthreads();
             if (kt + 1 == nk - 1) {
                 zero_tail(kt + 1);
@@ -913,32 +874,33 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
     }
 }
 
-template <int KIND, bool DUAL, int BK_, int NST, int BN_, int NWM_ = 2, int BM_ = 256>
-__global__ __launch_bounds__(128 * NWM_, (Geo<BK_, NST, BN_, NWM_, BM_>::WGS)) void grouped_gemm_kernel(GemmParams p) {
-    __shared__ uint4 lds_raw[gemm_lds_bytes<KIND, BK_, NST, BN_, NWM_, BM_>() / 16];
+template <int KIND, bool DUAL, int BK, int NST, int TILE>
+__global__ __launch_bounds__(256, (Geo<BK, NST, TILE>::WGS)) void grouped_gemm_kernel(GemmParams p) {
+    __shared__ uint4 lds_raw[gemm_lds_bytes<KIND, BK, NST, TILE>() / 16];
     // the experts' tiles, once per workgroup (before any tile's stores, so
     // the vector load of the offsets waits on nothing else)
     ExpertTiles et{};
-    if constexpr (!Traits<KIND>::group_k) et = expert_tiles<Geo<BK_, NST, BN_, NWM_, BM_>::BM>(p.offsets, p.E, threadIdx.x & 63);
-    if constexpr (persistent_tiles<KIND, BK_, BN_, NWM_, BM_>()) {
+    if constexpr (!Traits<KIND>::group_k) et = expert_tiles<TILE>(p.offsets, p.E, threadIdx.x & 63);
+    if constexpr (split_ring<KIND, TILE>()) {
         for (int vb = blockIdx.x; vb < p.vblocks; vb += gridDim.x)
-            grouped_gemm_tile<KIND, DUAL, BK_, NST, BN_, NWM_, BM_>(p, vb, et, lds_raw);
+            grouped_gemm_tile<KIND, DUAL, BK, NST, TILE>(p, vb, et, lds_raw);
     } else {
-        grouped_gemm_tile<KIND, DUAL, BK_, NST, BN_, NWM_, BM_>(p, blockIdx.x, et, lds_raw);
+        grouped_gemm_tile<KIND, DUAL, BK, NST, TILE>(p, blockIdx.x, et, lds_raw);
     }
 }
 
 // The split-K tail's second pass: tail tile j is the sum of its S partials
 // in part order, rounded once to bf16. Work items are (tile, 8-row slab);
 // thread t adds 8 columns of one row.
-template <int BK, int BN>
+template <int BK>
 __global__ __launch_bounds__(256) void split_fixup_kernel(GemmParams p) {
+    constexpr int BM = kLarge, BN = kLarge;
     const int ntn = (p.N + BN - 1) / BN, mtiles = act_mtiles(p);
     const SplitPlan sp = split_plan<BK>(p, mtiles * ntn);
     if (sp.S < 2) return;
     constexpr int kSlabs = BM / 8;
     const int tid = threadIdx.x;
-    const int rr = tid / (BN / 8), col = (tid % (BN / 8)) * 8;  // BN = 256: 8 rows x 32 lanes of 8 columns
+    const int rr = tid / (BN / 8), col = (tid % (BN / 8)) * 8;  // 8 rows x 32 lanes of 8 columns
     uint16_t* C = reinterpret_cast<uint16_t*>(p.c);
     for (int w = blockIdx.x; w < sp.R * kSlabs; w += gridDim.x) {
         const int j = w / kSlabs, slab = w % kSlabs;
@@ -982,27 +944,26 @@ __global__ __launch_bounds__(256) void split_fixup_kernel(GemmParams p) {
 //   to 0.72 us, mostly its LDS reads. K = 64 makes 128-byte row segments,
 //   which the CU's load path takes at twice the rate of 64-byte ones;
 //   128 x 128 weight-gradient tiles: 4 stages of K = 32, two workgroups per CU.
-template <int KIND, int TBM = BM, bool DEEP = false>
+template <int KIND, int TILE = kLarge, bool DEEP = false>
 struct Ring {
-    static constexpr bool split = split_ring<KIND, 64, TBM, 2, TBM>();
-    static constexpr bool k64 = TBM == 128 && !Traits<KIND>::group_k;
-    static constexpr int BK = split || k64 ? 64 : 32;
-    static constexpr int NST = split ? 3 : k64 && !DEEP ? 2 : 4;
+    static constexpr bool k64 = !Traits<KIND>::group_k;
+    static constexpr int BK = k64 ? 64 : 32;
+    static constexpr int NST = split_ring<KIND, TILE>() ? 3 : k64 && !DEEP ? 2 : 4;
 };
 
 // grid: the launch-order blocks of the tile map. Persistent kinds run
 // min(grid, CUs rounded down to a multiple of 8) workgroups over them.
-template <int KIND, bool DUAL, int TBM = BM, bool DEEP = false>
+template <int KIND, bool DUAL, int TILE = kLarge, bool DEEP = false>
 hipError_t launch_kind(const GemmParams& p, unsigned grid, hipStream_t s) {
-    using R = Ring<KIND, TBM, DEEP>;
+    using R = Ring<KIND, TILE, DEEP>;
     GemmParams q = p;
     q.vblocks = (int)grid;
     unsigned g = grid;
-    if constexpr (persistent_tiles<KIND, R::BK, TBM, 2, TBM>()) {
+    if constexpr (split_ring<KIND, TILE>()) {
         const unsigned cus = (unsigned)(cu_count() / 8 * 8);
         if (cus >= 8 && g > cus) g = cus;
     }
-    grouped_gemm_kernel<KIND, DUAL, R::BK, R::NST, TBM, 2, TBM><<<g, 256, 0, s>>>(q);
+    grouped_gemm_kernel<KIND, DUAL, R::BK, R::NST, TILE><<<g, 256, 0, s>>>(q);
     return hipGetLastError();
 }
 
@@ -1062,49 +1023,48 @@ GemmTile gemm_tile(GemmKind kind, const GemmParams& p) {
 }
 
 hipError_t launch_gemm_tile(GemmKind kind, bool dual, const GemmParams& p, GemmTile tile, hipStream_t s) {
-    const int bn = tile.m, bm = tile.m;
+    const int m = tile.m;
     if (p.N % 8 != 0 || p.N <= 0) return hipErrorInvalidValue;
-    if (bm != 256 && bm != 128) return hipErrorInvalidValue;
+    if (m != 256 && m != 128) return hipErrorInvalidValue;
     const bool group_k = kind == GEMM_DW_DOWN || kind == GEMM_DW_UP;
     const bool fp4 = kind == GEMM_UP_FP4 || kind == GEMM_DOWN_FP4;
-    if (tile.deep && (bm != 128 || group_k)) return hipErrorInvalidValue;
-    if (fp4 && bm != 256) return hipErrorInvalidValue;
-    const int64_t ntn = (p.N + bn - 1) / bn;
+    if (tile.deep && (m != 128 || group_k)) return hipErrorInvalidValue;
+    if (fp4 && m != 256) return hipErrorInvalidValue;
+    const int64_t ntn = (p.N + m - 1) / m;
     int64_t grid;
     if (group_k) {
         if (p.M % 8 != 0 || p.M <= 0) return hipErrorInvalidValue;
         if (p.m_out > p.M || p.n_out > p.N || p.M - p.m_out >= 64 || p.N - p.n_out >= 64 || p.ldc < p.n_out)
             return hipErrorInvalidValue;
         // whole rounds of 8 XCDs x 32 workgroups keep the block -> tile map a bijection
-        grid = ((int64_t)p.E * ((p.M + bm - 1) / bm) * ntn + 255) / 256 * 256;
+        grid = ((int64_t)p.E * ((p.M + m - 1) / m) * ntn + 255) / 256 * 256;
     } else {
         if (p.K % 64 != 0) return hipErrorInvalidValue;
-        // sum_e ceil(cnt_e / bm) <= ceil(slots / bm) + E - 1
-        const int64_t tiles = ((int64_t)(p.slots + bm - 1) / bm + p.E) * ntn;
+        // sum_e ceil(cnt_e / m) <= ceil(slots / m) + E - 1
+        const int64_t tiles = (((int64_t)p.slots + m - 1) / m + p.E) * ntn;
         grid = tiles >= 8 * 256 ? (tiles + 255) / 256 * 256 : (tiles + 7) / 8 * 8;  // whole rounds, or eight equal runs
     }
-    const GemmParams& q = p;
-    // split-K tail (GEMM_DOWN / GEMM_DX on 256-column tiles): its parts are
+    // split-K tail (GEMM_DOWN / GEMM_DX on 256 x 256 tiles): its parts are
     // the workgroups after the whole rounds, at most `resident` of them.
-    const bool split = (kind == GEMM_DOWN || kind == GEMM_DX) && bm == 256 && p.part != nullptr &&
+    const bool split = (kind == GEMM_DOWN || kind == GEMM_DX) && m == 256 && p.part != nullptr &&
                        p.resident > 0 && p.resident % 256 == 0;
     if (split) grid += p.resident;
     if (grid <= 0) return hipSuccess;
     if (grid > 0x7fffffff) return hipErrorInvalidValue;
     const unsigned g = (unsigned)grid;
     if (split) {
-        hipError_t err = kind == GEMM_DOWN ? launch_kind<GEMM_DOWN, false>(q, g, s) : launch_kind<GEMM_DX, false>(q, g, s);
+        hipError_t err = kind == GEMM_DOWN ? launch_kind<GEMM_DOWN, false>(p, g, s) : launch_kind<GEMM_DX, false>(p, g, s);
         if (err != hipSuccess) return err;
         static_assert(Ring<GEMM_DOWN>::BK == Ring<GEMM_DX>::BK, "one split plan for DOWN and DX");
         // 4 workgroups per CU: the (tile, 8-row slab) items are short and latency-bound
-        split_fixup_kernel<Ring<GEMM_DOWN>::BK, 256><<<p.resident * 4, 256, 0, s>>>(q);
+        split_fixup_kernel<Ring<GEMM_DOWN>::BK><<<p.resident * 4, 256, 0, s>>>(p);
         return hipGetLastError();
     }
 #define TMT_ACT(KIND_, DUAL_)                                   \
-    (bm == 256    ? launch_kind<KIND_, DUAL_>(q, g, s)          \
-     : !tile.deep ? launch_kind<KIND_, DUAL_, 128>(q, g, s)     \
-                  : launch_kind<KIND_, DUAL_, 128, true>(q, g, s))
-#define TMT_DW(KIND_) (bm == 256 ? launch_kind<KIND_, false>(q, g, s) : launch_kind<KIND_, false, 128>(q, g, s))
+    (m == 256     ? launch_kind<KIND_, DUAL_>(p, g, s)          \
+     : !tile.deep ? launch_kind<KIND_, DUAL_, 128>(p, g, s)     \
+                  : launch_kind<KIND_, DUAL_, 128, true>(p, g, s))
+#define TMT_DW(KIND_) (m == 256 ? launch_kind<KIND_, false>(p, g, s) : launch_kind<KIND_, false, 128>(p, g, s))
     switch (kind) {
         case GEMM_UP: return dual ? TMT_ACT(GEMM_UP, true) : TMT_ACT(GEMM_UP, false);
         case GEMM_DOWN: return TMT_ACT(GEMM_DOWN, false);
@@ -1112,8 +1072,8 @@ hipError_t launch_gemm_tile(GemmKind kind, bool dual, const GemmParams& p, GemmT
         case GEMM_DX: return TMT_ACT(GEMM_DX, false);
         case GEMM_DW_DOWN: return TMT_DW(GEMM_DW_DOWN);
         case GEMM_DW_UP: return TMT_DW(GEMM_DW_UP);
-        case GEMM_UP_FP4: return dual ? launch_kind<GEMM_UP_FP4, true>(q, g, s) : launch_kind<GEMM_UP_FP4, false>(q, g, s);
-        case GEMM_DOWN_FP4: return launch_kind<GEMM_DOWN_FP4, false>(q, g, s);
+        case GEMM_UP_FP4: return dual ? launch_kind<GEMM_UP_FP4, true>(p, g, s) : hipErrorInvalidValue;
+        case GEMM_DOWN_FP4: return launch_kind<GEMM_DOWN_FP4, false>(p, g, s);
         default: return hipErrorInvalidValue;
     }
 #undef TMT_ACT
