@@ -1284,13 +1284,9 @@ hipError_t launch_scatter(const ScatterParams& p, hipStream_t s) {
     const bool router = p.dlogits != nullptr && p.E > 1;
     const bool ln = p.ln_S != nullptr;
     if (ln && p.d > kLnFusedMaxD) return hipErrorInvalidValue;
-    const int rows = scatter_ln_rows(p.T);  // LayerNorm variants
     const bool wlds = router && router_wr_in_lds(p.E, p.d);  // Wr staged in LDS
     const size_t wr_lds = wlds ? (size_t)p.E * p.d * 2 : 0;
-    size_t lds = router ? wr_lds + (size_t)rows * p.E * 4 : 0;
-    if (ln && !(wlds && p.E >= kRedOnWrExperts)) lds += (size_t)3 * 2 * p.d * 4;
-    const int ni = ln ? (p.d + 511) / 512 : 0;
-    if (ni == 0) {
+    if (!ln) {
         // router variant: fewer rows per workgroup while that keeps the grid
         // under 512 workgroups (small T: each wave's chain of chunk loads is
         // the time, so more, shorter workgroups finish sooner)
@@ -1319,6 +1315,9 @@ hipError_t launch_scatter(const ScatterParams& p, hipStream_t s) {
         }
         return hipGetLastError();
     }
+    const int ni = (p.d + 511) / 512, rows = scatter_ln_rows(p.T);
+    size_t lds = router ? wr_lds + (size_t)rows * p.E * 4 : 0;
+    if (!(wlds && p.E >= kRedOnWrExperts)) lds += (size_t)3 * 2 * p.d * 4;
     if (!router) return launch_scatter_ni<false, false>(p, ni, rows, lds, s);
     if (p.K <= 4 && ni <= 2) {
         // two rows per wave in flight (scatter_ln2_kernel)
