@@ -640,8 +640,11 @@ size_t stream_lds_rt(bool halves, bool dual, int rb, int nw, int ntile, int spli
 // stream is a quarter of the bf16 one, so a decode step is bound by the
 // memory round trips of a workgroup (tables, then codes and activations, then
 // the reduction) more than by bytes: every code and scale load of a
-// workgroup's columns is issued at once, and the grid covers the chip in one
-// round. Workgroup: 64 output columns and up to 16 RBP rows of one expert;
+// workgroup's columns is issued at once. With one chunk per wave at 16 waves
+// (the DOWN below) the kernel takes 90 VGPRs, five waves per SIMD, so one
+// workgroup fits a CU: at T = 8 the about 21 experts with rows make 336
+// workgroups of DOWN, a round of 256 and a second one a third full.
+// Workgroup: 64 output columns and up to 16 RBP rows of one expert;
 // wave w reduces the 256-element chunks w, w + nw, ... of K (ONE: one chunk
 // per wave). Lane (g, li) holds, per 16-column tile, the codes of
 // k = 256 q + 128 c + 32 g .. + 31 (c = 0, 1) of column li: one 16-byte load
@@ -650,7 +653,7 @@ size_t stream_lds_rt(bool halves, bool dual, int rb, int nw, int ntile, int spli
 // block's scale bytes one whole 64-byte segment ([K/32][N] layout). The codes
 // are expanded to bf16 in registers (exact, as in gemm.hip) once per chunk
 // for the RBP row blocks that use them.
-// Measured (d = 1024, h = 4096, E = 32, top-4, T = 8; about 92 MB of the
+// Measured (d = 1024, h = 4096, E = 32, top-4, T = 8; about 94 MB of the
 // picked experts' codes and scales per step), against the 256 x 256 tiles of
 // gemm.hip: UP 62.8 -> 15.6 us, DOWN 102.8 -> 16.7 us, step 169.6 -> 46.1 us.
 constexpr int kFp4Cols = 64;
@@ -822,7 +825,7 @@ template <int KIND, int RBP>
 hipError_t launch_fp4_rows(const GemmParams& p, int T, hipStream_t s) {
     constexpr int RB = 16 * RBP;
     const int nchunk = (p.K + 255) / 256;
-    const int most = RBP == 1 && nchunk <= 16 ? 16 : 8;  // waves (16 only with one chunk each: 128 VGPRs)
+    const int most = RBP == 1 && nchunk <= 16 ? 16 : 8;  // waves (16 only with one chunk each, within 128 VGPRs)
     const int nw = std::min(nchunk, most);
     // self_dispatch: the expert's row blocks by index; otherwise the list of
     // (expert, row block) from the offsets, at most slots / RB + E entries
