@@ -24,12 +24,11 @@
  * the caller's tensors directly and every device pointer must be 16-byte
  * aligned. Other widths (TMT's own tests run dim 16 and 32) run on
  * zero-padded copies at the widths rounded up to 64, kept in the handle's
- * shared workspace: each call copies its operands in and Y and dX out
- * (a few extra small kernels; the weight gradients are written in place),
- * and pointers need only their natural alignment (2 bytes for bf16, 4 for
- * fp32). Zero columns add exact zeros, so
- * the routing is the same as at the caller's width. The MXFP4 formats keep
- * d and hidden multiples of 64.
+ * shared workspace: each call copies its operands in and Y, dX and dWr out
+ * (a few extra small kernels; the expert weight gradients are written in
+ * place), and pointers need only their natural alignment (2 bytes for bf16,
+ * 4 for fp32). Zero columns add exact zeros, so the routing is the same as at
+ * the caller's width. The MXFP4 formats keep d and hidden multiples of 64.
  *
  * Every function returns TMT_MOE_OK (0) or a negative error code and never
  * exits the process; tmt_moe_last_error() gives a thread-local message.

@@ -350,10 +350,10 @@ __device__ __forceinline__ void grouped_gemm_tile(const GemmParams& p, const int
         // come in descending-count order. With G % 8 as the XCD, an expert
         // whose groups fill half of the XCDs sends every following expert to
         // the same halves in turn (c3: 74K against 57K slots per XCD).
-        //  * 128-column tiles (two workgroups per CU): round r hands its 8
+        //  * 128 x 128 tiles (two workgroups per CU): round r hands its 8
         //    groups of 32 tiles to the XCDs in snake order (reversed on odd
         //    rounds), which keeps every XCD's sum of counts near the mean;
-        //  * 256-column tiles (one per CU): groups of 16 tiles, two per XCD
+        //  * 256 x 256 tiles (one per CU): groups of 16 tiles, two per XCD
         //    and round, paired heaviest with lightest (XCD x runs groups
         //    16r + x and 16r + 15 - x). With 32-tile groups the XCD holding
         //    the heaviest expert's group could not be balanced.

@@ -693,7 +693,7 @@ bool dx_transposed(const tmt_moe* m, int T) {
 // internal widths, and so has W_up unless dx_transposed; the weight gradients
 // are the caller's (dWr: internal width). With `ln`, dX is the gradient
 // at the LayerNorm output: for d <= kLnFusedMaxD the scatter consumes it in
-// registers (dX is not written), otherwise it lands in dX and the two-pass
+// registers (dX is not written), otherwise it lands in dX and the separate
 // LayerNorm backward follows.
 int run_backward(tmt_moe* m, hipStream_t s, const uint16_t* dY, const uint16_t* X,
                  const uint16_t* Wr, const uint16_t* const* W_up, const uint16_t* const* W_down,
@@ -947,7 +947,7 @@ int create_handle(const tmt_moe_desc* desc, void* workspace, size_t workspace_by
     m->user = *desc;
     m->hn = m->desc.hidden > 0 ? m->desc.hidden : m->desc.d;
     if (is_padded(*desc)) {
-        // operands are read element by element into the padded copies
+        // operands are copied into the padded ones from any element's address
         m->align_bf16 = 2;
         m->align_f32 = 4;
     }
