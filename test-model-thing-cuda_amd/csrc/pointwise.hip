@@ -1066,8 +1066,9 @@ __global__ __launch_bounds__(kThreads) void scatter_ln2_kernel(ScatterParams p, 
 // rows in a chain of load round trips, so a small batch finishes sooner on
 // many short workgroups: T = 1024, d = 256 took 19.9 us on 16 workgroups of 64
 // rows and 3.0 us more for the router gradient's second pass, 5.9 us on 128 of
-// 8 with that pass riding along (kernel trace). The block's step at T = 4096, d = 1024, E = 16: 239 us below 128 workgroups,
-// 230 below 256, 226.5 below 512 and below 1024.
+// 8 with that pass riding along (kernel trace). The block's step at T = 4096,
+// d = 1024, E = 16: 239 us below 128 workgroups, 230 below 256, 226.5 below
+// 512 and below 1024.
 constexpr int kScatterLnRows = 64, kScatterLnRowsMin = 8, kScatterLnBlocks = 512;
 static int scatter_ln_rows(int T) {
     int rows = kScatterLnRows;
