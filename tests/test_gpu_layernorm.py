@@ -128,7 +128,7 @@ def check_all(g, r, E, h):
 
 
 @pytest.mark.parametrize("T,d,E,K,h", [
-    (300, 256, 4, 2, 1024),    # a few 64-row workgroups of the fused dGamma/dBeta partials
+    (300, 256, 4, 2, 1024),    # 38 workgroups of 8 rows in the fused scatter, the last one half full
     (1237, 384, 8, 2, 256),    # ragged T, d not a multiple of 512
     (520, 1088, 4, 2, 128),    # d > 512: three row passes per lane, the last partial
     (520, 1088, 16, 4, 128),   # LayerNorm inside the router: 4 chunk slots, the third partial, the fourth empty
@@ -137,7 +137,7 @@ def check_all(g, r, E, h):
     (5, 192, 5, 2, 320),       # decode-sized: fused router, weight-streaming GEMMs
     (64, 1024, 16, 4, 512),    # largest decode batch, c3 width
     (2100, 2048, 12, 2, 128),  # widest row of the scatter-fused backward (4 passes per lane)
-    (300, 2560, 4, 2, 128),    # d > 2048: separate two-pass LayerNorm backward
+    (300, 2560, 4, 2, 128),    # d > 2048: separate LayerNorm backward
     (200, 2048, 32, 4, 128),   # E*d beyond the LDS-staged router: fused scatter reads Wr from memory
     (160, 2560, 16, 4, 0),     # the same on the separate LayerNorm backward, reference experts
 ])
@@ -162,6 +162,25 @@ def test_layernorm_block_short_router_blocks(orc, T, d, E, K):
     """The LayerNorm in a router that takes fewer rows per wave."""
     say(f"LayerNorm + router blocks T={T} d={d} E={E} K={K}")
     case = make_case(T, d, E, K, 0, seed=T + E)
+    S, gamma, beta = ln_inputs(case["X"], seed=T)
+    Y0 = bf16_bits(np.zeros((T, d), np.float32))
+    check_all(run_gpu_ln(case, S, gamma, beta, K, 0, Y0, 0.01, 0.001),
+              oracle_ln(orc, case, S, gamma, beta, K, 0, Y0, 0.01, 0.001), E, 0)
+
+
+@pytest.mark.parametrize("T,d,E,K", [
+    (4090, 64, 4, 2),    # 8 rows per workgroup, 512 workgroups, the last one two rows long
+    (8195, 64, 4, 2),    # 16 rows
+    (16390, 64, 4, 2),   # 32 rows
+    (32710, 64, 4, 2),   # 64 rows
+    (8195, 128, 8, 6),   # six picks: one row per wave at a time, 16 rows
+    (8195, 1088, 12, 2), # three chunks per row, dGamma / dBeta sums over Wr's LDS, 16 rows
+])
+def test_layernorm_block_scatter_blocks(orc, T, d, E, K):
+    """The fused LayerNorm backward at every workgroup length of the scatter
+    (8 to 64 rows), its last workgroup short."""
+    say(f"LayerNorm + scatter blocks T={T} d={d} E={E} K={K}")
+    case = make_case(T, d, E, K, 0, seed=T + K)
     S, gamma, beta = ln_inputs(case["X"], seed=T)
     Y0 = bf16_bits(np.zeros((T, d), np.float32))
     check_all(run_gpu_ln(case, S, gamma, beta, K, 0, Y0, 0.01, 0.001),

@@ -167,7 +167,7 @@ def test_width_layernorm_block(orc, T, d, E, K, h):
 @pytest.mark.parametrize("T,d", [(9, 17), (300, 100), (64, 16), (5, 3)])
 def test_width_standalone_layernorm(orc, T, d):
     """tmt_moe_layernorm_forward / _backward at widths that are not multiples
-    of 8: element accesses, same summation order as the oracle."""
+    of 8: unaligned pieces, same summation order as the oracle."""
     say(f"standalone LayerNorm T={T} d={d}")
     rng = np.random.default_rng(T * 31 + d)
     X = bf16_bits(rng.standard_normal((T, d)).astype(np.float32))
